@@ -71,7 +71,8 @@ typedef enum splosh_kernel {
                                    rows 0..63 and the rest as two calls of the above (without the
                                    emit); more: PREFILL for tiled weights with lda % 8 == 0 and
                                    ldc % 4 == 0, else TILE; SCALAR for operands no other kernel
-                                   takes */
+                                   takes. A row-major weight of one or two rows, or of few outputs
+                                   (rows.hip), takes a latency-shaped kernel of its own first */
     SPLOSH_KERNEL_STREAM = 1,   /* weight streaming on raw codes: the every-CU decode kernel for
                                    1-4 rows of tiled weights (with a workspace it splits the last
                                    round of row blocks over K, so every CU gets the same share),

@@ -102,6 +102,11 @@ int q4_gemm_impl(const splosh_q4_weight *w, const splosh_q4_weight *up, const ui
     const bool eligible = q4_stream_eligible(*w, a, lda) && (!up || q4_stream_eligible(*up, a, lda));
     const bool wide16 = eligible && aligned(w->packed, 16) && (!up || aligned(up->packed, 16)) &&
                         (w->order == SPLOSH_Q4_TILED128 || w->row_stride_words % 4 == 0);
+    // Row-major weights of one or two rows, or of few outputs: latency alone bounds them.
+    if (kernel == SPLOSH_KERNEL_AUTO && !up && !emit && wide16 && w->order == SPLOSH_Q4_ROW_MAJOR &&
+        splosh::rows_fit(rows, w->rows, w->inner, lda))
+        return hip_status(splosh::launch_q4_rows(*w, a, lda, out, ldc, out_dtype, residual, rows, stream),
+                          "q4 rows launch");
     // 65..128 rows under AUTO: rows 0..63 and the rest as two calls of the M <= 64 kernels, one after
     // the other on the stream (the workspace's counters are zero again between them). Measured at
     // K5120 -> 2 x N17408 (gate+up) and K17408 -> N5120, against the one call on the tile or
