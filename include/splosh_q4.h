@@ -64,9 +64,10 @@ typedef enum splosh_dtype { SPLOSH_F32 = 0, SPLOSH_BF16 = 1 } splosh_dtype;
 /* Kernel choice (the reference selects kernels through SPLOSH_* environment variables,
  * Runtime/Engine.swift:380-440; here the caller names one, or AUTO picks by rows). */
 typedef enum splosh_kernel {
-    SPLOSH_KERNEL_AUTO = 0,     /* 1..4 rows of tiled weights whose staged activation rows fit 80 KB
-                                   (one or two rows up to K of about 18700, four up to about 9100):
-                                   STREAM; else up to 64: DEQUANT (a single weight of at least two
+    SPLOSH_KERNEL_AUTO = 0,     /* one or two rows of tiled weights whose staged activation rows fit
+                                   80 KB (K up to about 18700): STREAM; 3..16 rows of tiled weights,
+                                   and up to 32 where it wins (skinny.hip), the raw-code MFMA kernel
+                                   without a barrier in its loop; else up to 64: DEQUANT (a single weight of at least two
                                    64-column bands a CU as the pair of its column halves); 65..128:
                                    rows 0..63 and the rest as two calls of the above (without the
                                    emit); more: PREFILL for tiled weights with lda % 8 == 0 and
@@ -201,8 +202,8 @@ int splosh_q4_gemm_noalloc(const splosh_q4_weight *w, const uint16_t *a, int64_t
  * 57-62; the GEMMs at Engine.swift:1131-1140). out_i = a @ dequant(w_i)^T for i < count
  * (count <= SPLOSH_MAX_GROUP), each into its own output (row stride ldcs[i], out_dtype), no
  * residual. All weights share inner. Up to 64 rows with TILED128 weights (rows % 64 == 0) the
- * group is one launch of the M <= 64 kernel over the weights' joined column bands, split over the
- * CUs as one call (workspace: splosh_workspace_bytes(rows, sum of the weights' rows, inner));
+ * group is one launch of the M <= 64 kernel (at few rows the one AUTO gives a single weight from
+ * three rows) over the weights' joined column bands, split over the CUs as one call (workspace: splosh_workspace_bytes(rows, sum of the weights' rows, inner));
  * otherwise each weight is its own splosh_q4_gemm call, same results to the path's tolerance. */
 #define SPLOSH_MAX_GROUP 8
 int splosh_q4_gemm_group(const splosh_q4_weight *weights, int count, const uint16_t *a, int64_t lda,

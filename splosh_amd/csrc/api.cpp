@@ -123,6 +123,14 @@ int q4_gemm_impl(const splosh_q4_weight *w, const splosh_q4_weight *up, const ui
                             res ? res + 64 * ldc * esize : nullptr, rows - 64, kernel, workspace, workspace_bytes,
                             stream);
     }
+    // 3..32 rows of tiled weights (one and two rows: the decode kernel below, unless their staged
+    // activations do not fit it).
+    if (kernel == SPLOSH_KERNEL_AUTO && wide16 && w->order == SPLOSH_Q4_TILED128 &&
+        (rows >= 3 || !splosh::decode_fits(rows, w->rows, w->inner, w->order)) &&
+        splosh::skinny_fits(rows, w->rows, w->inner, lda, up != nullptr))
+        return hip_status(splosh::launch_q4_skinny(*w, up, a, lda, out, ldc, out_dtype, residual, rows, workspace,
+                                                   workspace ? workspace_bytes : 0, stream),
+                          "q4 skinny launch");
     const bool tile_ok = wide16 && splosh::tile_fits(rows, w->rows, lda, w->row_stride_words);
     const bool mma_ok = wide16 && splosh::mma_fits(rows, w->rows, w->inner, w->row_stride_words, lda);
     const bool prefill_ok = wide16 && !up && w->order == SPLOSH_Q4_TILED128 && aligned(out, 16) &&
@@ -403,9 +411,11 @@ size_t splosh_workspace_bytes(int64_t rows, int64_t columns, int64_t inner) {
     const size_t prefill = rows > 64 && columns % 128 == 0 ? splosh::prefill_workspace_bytes(rows, 2 * columns, groups) : 0;
     const size_t gguf = inner % 64 == 0 ? splosh::gguf_tile_workspace_bytes(rows, columns, inner) : 0;
     const size_t decode = splosh::decode_workspace_bytes(rows, columns, inner, 2);
+    const size_t skinny = splosh::skinny_workspace_bytes(rows, columns, inner, 2);
     const size_t q5k_decode = splosh::q5k_decode_workspace_bytes(rows, columns, inner);
     size_t need = tile > mma ? tile : mma;
     need = need > decode ? need : decode;
+    need = need > skinny ? need : skinny;
     need = need > q5k_decode ? need : q5k_decode;
     need = need > prefill ? need : prefill;
     return need > gguf ? need : gguf;
@@ -507,6 +517,10 @@ int splosh_q4_gemm_group(const splosh_q4_weight *weights, int count, const uint1
                 return st;
         return ok();
     }
+    if (kernel == SPLOSH_KERNEL_AUTO && splosh::skinny_fits(rows, columns, weights[0].inner, lda, false))
+        return hip_status(splosh::launch_q4_skinny_group(weights, count, outs, ldcs, a, lda, out_dtype, rows, workspace,
+                                                         workspace ? workspace_bytes : 0, stream),
+                          "q4 grouped skinny launch");
     const splosh::MmaPlan plan =
         splosh::plan_mma(rows, columns, weights[0].inner / kGroupSize, false, workspace ? workspace_bytes : 0);
     return hip_status(splosh::launch_q4_mma_group(plan, weights, count, outs, ldcs, a, lda, out_dtype, rows, workspace,

@@ -67,6 +67,18 @@ hipError_t launch_q4_decode(const splosh_q4_weight &w, const splosh_q4_weight *u
                             void *out, int64_t ldc, int out_dtype, const void *residual, int64_t rows,
                             void *workspace, size_t workspace_bytes, hipStream_t stream);
 
+// The raw-code MFMA kernel for a few rows of tiled weights (skinny.hip): 32 output columns a
+// workgroup, no barrier in its loop. With a workspace of skinny_workspace_bytes (zero: not needed)
+// it splits K where the blocks do not fill the CUs evenly.
+bool skinny_fits(int64_t rows, int64_t columns, int64_t inner, int64_t lda, bool pair);
+size_t skinny_workspace_bytes(int64_t rows, int64_t columns, int64_t inner, int nw);
+hipError_t launch_q4_skinny(const splosh_q4_weight &w, const splosh_q4_weight *up, const uint16_t *a, int64_t lda,
+                            void *out, int64_t ldc, int out_dtype, const void *residual, int64_t rows, void *workspace,
+                            size_t workspace_bytes, hipStream_t stream);
+hipError_t launch_q4_skinny_group(const splosh_q4_weight *w, int count, void *const *outs, const int64_t *ldcs,
+                                  const uint16_t *a, int64_t lda, int out_dtype, int64_t rows, void *workspace,
+                                  size_t workspace_bytes, hipStream_t stream);
+
 // The dequant-to-bf16 weight-streaming MFMA kernel for up to 64 rows (mma.hip). Split K over
 // workgroups (stream-K) uses a caller workspace of mma_workspace_bytes(); without one every band
 // is computed whole by one workgroup.
