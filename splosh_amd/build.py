@@ -17,7 +17,7 @@ ROOT = PKG.parent
 CSRC = PKG / "csrc"
 BUILD = PKG / "_build"
 LIB = PKG / "libsplosh_q4.so"
-SOURCES = ["api.cpp", "q4_basic.hip", "stream.hip", "lanes.hip", "rows.hip", "decode.hip", "skinny.hip", "mma.hip", "tile.hip", "prefill.hip", "q5k.hip", "q5k_decode.hip", "operand.hip", "gguf_native.hip", "gguf_tile.hip"]
+SOURCES = ["api.cpp", "q4_basic.hip", "stream.hip", "lanes.hip", "rows.hip", "decode.hip", "skinny.hip", "skinny_gguf.hip", "mma.hip", "tile.hip", "prefill.hip", "q5k.hip", "q5k_decode.hip", "operand.hip", "gguf_native.hip", "gguf_tile.hip"]
 PROBE_LIB = PKG / "libsplosh_probe.so"
 PROBE_SOURCES = ["bench/probe.hip"]
 

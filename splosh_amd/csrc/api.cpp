@@ -412,10 +412,12 @@ size_t splosh_workspace_bytes(int64_t rows, int64_t columns, int64_t inner) {
     const size_t gguf = inner % 64 == 0 ? splosh::gguf_tile_workspace_bytes(rows, columns, inner) : 0;
     const size_t decode = splosh::decode_workspace_bytes(rows, columns, inner, 2);
     const size_t skinny = splosh::skinny_workspace_bytes(rows, columns, inner, 2);
+    const size_t gguf_skinny = splosh::gguf_skinny_workspace_bytes(rows, columns, inner);
     const size_t q5k_decode = splosh::q5k_decode_workspace_bytes(rows, columns, inner);
     size_t need = tile > mma ? tile : mma;
     need = need > decode ? need : decode;
     need = need > skinny ? need : skinny;
+    need = need > gguf_skinny ? need : gguf_skinny;
     need = need > q5k_decode ? need : q5k_decode;
     need = need > prefill ? need : prefill;
     return need > gguf ? need : gguf;
@@ -658,6 +660,12 @@ static int gguf_gemm(const splosh_q5k_weight *w_in, bool fifth, const uint16_t *
     const bool prefill_ok = eligible && lda % 8 == 0 && aligned(a, 16) && aligned(out, 16) &&
                             (!residual || aligned(residual, 16)) &&
                             splosh::q5k_prefill_fits(rows, w->rows, w->inner, lda, ldc);
+    if (kernel == SPLOSH_KERNEL_AUTO && mma_ok &&
+        splosh::gguf_skinny_fits(fifth ? 13 : 12, rows, w->rows, w->inner, lda, w->rows * (w->inner / 32) * 16))
+        return hip_status(splosh::launch_gguf_skinny(fifth ? 13 : 12, w->plane0, w->plane1, w->meta, w->rows, w->inner, a,
+                                                     lda, out, ldc, out_dtype, residual, rows, workspace,
+                                                     workspace ? workspace_bytes : 0, stream),
+                          "gguf skinny launch");
     int choice = kernel;
     if (kernel == SPLOSH_KERNEL_AUTO) {
         if (!eligible) choice = SPLOSH_KERNEL_SCALAR;
@@ -800,7 +808,8 @@ static int gguf_native_gemm(int gguf_type, const uint8_t *native, int64_t rows, 
     // 47, IQ3_S 42, IQ4_NL 27, IQ4_XS 30); the streaming kernel at four rows Q8_0 31, Q6_K 35, Q3_K
     // 32, IQ3_S 31, IQ4_NL 29, IQ4_XS 29, at five Q6_K 45, Q3_K 43, IQ3_S 43, at six Q3_K 47, at
     // three IQ4_NL 26. Where the MFMA kernel does not fit (K % 256 != 0), the streaming kernel
-    // serves up to eight rows and the LDS-tiled kernel above. (A development override of the
+    // serves up to eight rows and the LDS-tiled kernel above. Up to 32 rows the barrier-free kernel of
+    // skinny_gguf.hip comes first where it is the faster. (A development override of the
     // prefill threshold, read once.)
     static const int64_t prefill_rows = [] {
         const char *e = getenv("SPLOSH_GGUF_PREFILL_ROWS");
@@ -823,11 +832,17 @@ static int gguf_native_gemm(int gguf_type, const uint8_t *native, int64_t rows, 
                                 ldc, out_dtype, res ? res + 64 * ldc * esize : nullptr, m - 64, workspace,
                                 workspace_bytes, stream, key_heads);
     }
-    const bool mma = !prefill && m > stream_max && splosh::gguf_mma_fits(gguf_type, m, rows, inner, lda);
-    const bool tile = !prefill && !mma && m > 8 && splosh::gguf_tile_fits(m, rows, inner, lda);
+    int elems = 0, bytes = 0;
+    splosh::gguf_native_block(base_type, &elems, &bytes);
+    const int64_t stored = (gguf_type & SPLOSH_GGUF_ROWS32) ? (rows + 31) / 32 * 32 : rows;
+    // (A head-ordered call the streaming kernel takes stays there: it needs no workspace.)
+    const bool skinny = !(ho.on() && m <= stream_max) &&
+                        splosh::gguf_skinny_fits(gguf_type, m, rows, inner, lda, stored * (inner / elems * bytes));
+    const bool mma = !prefill && !skinny && m > stream_max && splosh::gguf_mma_fits(gguf_type, m, rows, inner, lda);
+    const bool tile = !prefill && !skinny && !mma && m > 8 && splosh::gguf_tile_fits(m, rows, inner, lda);
     // The streaming kernels read the activations through head_group(); the other kernels get a
     // permuted copy.
-    if (ho.on() && (prefill || mma || tile)) {
+    if (ho.on() && (prefill || skinny || mma || tile)) {
         if ((st = head_copy(ho, &a, &lda, m, inner, workspace, &workspace_bytes, stream))) return st;
         if (workspace_bytes == 0) workspace = nullptr;
     }
@@ -837,6 +852,11 @@ static int gguf_native_gemm(int gguf_type, const uint8_t *native, int64_t rows, 
                                                       residual, m, workspace, stream),
                           "gguf prefill launch");
     }
+    if (skinny)
+        return hip_status(splosh::launch_gguf_skinny(gguf_type, native, nullptr, nullptr, rows, inner, a, lda, out, ldc,
+                                                     out_dtype, residual, m, workspace,
+                                                     workspace ? workspace_bytes : 0, stream),
+                          "gguf skinny launch");
     if (mma) {
         const splosh::MmaPlan plan =
             splosh::plan_mma(m, rows, inner / 256, false, workspace ? workspace_bytes : 0, 256);

@@ -79,6 +79,15 @@ hipError_t launch_q4_skinny_group(const splosh_q4_weight *w, int count, void *co
                                   const uint16_t *a, int64_t lda, int out_dtype, int64_t rows, void *workspace,
                                   size_t workspace_bytes, hipStream_t stream);
 
+// The same shape for GGUF weights (skinny_gguf.hip): type a native-block id with its layout flag, or
+// 13 / 12 for Q5_K / Q4_K planes (w = plane0). weight_bytes: of the native blocks or plane0.
+bool gguf_skinny_fits(int type, int64_t rows, int64_t columns, int64_t inner, int64_t lda, int64_t weight_bytes);
+size_t gguf_skinny_workspace_bytes(int64_t rows, int64_t columns, int64_t inner);
+hipError_t launch_gguf_skinny(int type, const uint8_t *w, const uint8_t *plane1, const uint8_t *meta, int64_t columns,
+                              int64_t inner, const uint16_t *a, int64_t lda, void *out, int64_t ldc, int out_dtype,
+                              const void *residual, int64_t rows, void *workspace, size_t workspace_bytes,
+                              hipStream_t stream);
+
 // The dequant-to-bf16 weight-streaming MFMA kernel for up to 64 rows (mma.hip). Split K over
 // workgroups (stream-K) uses a caller workspace of mma_workspace_bytes(); without one every band
 // is computed whole by one workgroup.
