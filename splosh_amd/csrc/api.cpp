@@ -407,8 +407,13 @@ size_t splosh_workspace_bytes(int64_t rows, int64_t columns, int64_t inner) {
     const size_t tile = splosh::tile_workspace_bytes(rows, columns, groups, true);
     // (65..128 rows run as two calls of at most 64 rows.)
     const size_t mma = rows <= 128 ? splosh::mma_workspace_bytes(rows < 64 ? rows : 64, columns, groups, true) : 0;
-    // (2 columns: the fused gate+up plans its tiles over both weights' columns.)
-    const size_t prefill = rows > 64 && columns % 128 == 0 ? splosh::prefill_workspace_bytes(rows, 2 * columns, groups) : 0;
+    // (And twice the columns: the fused gate+up plans its tiles over both weights' columns.)
+    size_t prefill = 0;
+    if (rows > 64 && columns % 128 == 0) {
+        const size_t one = splosh::prefill_workspace_bytes(rows, columns, groups);
+        const size_t two = splosh::prefill_workspace_bytes(rows, 2 * columns, groups);
+        prefill = one > two ? one : two;
+    }
     const size_t gguf = inner % 64 == 0 ? splosh::gguf_tile_workspace_bytes(rows, columns, inner) : 0;
     const size_t decode = splosh::decode_workspace_bytes(rows, columns, inner, 2);
     const size_t skinny = splosh::skinny_workspace_bytes(rows, columns, inner, 2);
@@ -501,6 +506,7 @@ int splosh_q4_gemm_group(const splosh_q4_weight *weights, int count, const uint1
     int64_t columns = 0;
     bool joined = rows <= 64 && (kernel == SPLOSH_KERNEL_AUTO || kernel == SPLOSH_KERNEL_DEQUANT) && lda % 8 == 0 &&
                   aligned(a, 16);
+    bool wide = rows > 64 && kernel == SPLOSH_KERNEL_AUTO && lda % 8 == 0 && aligned(a, 16);
     for (int i = 0; i < count; ++i) {
         const splosh_q4_weight *w = &weights[i];
         if ((st = check_q4_weight(w, "weight"))) return st;
@@ -508,7 +514,29 @@ int splosh_q4_gemm_group(const splosh_q4_weight *weights, int count, const uint1
         if ((st = check_io(a, lda, outs[i], ldcs[i], out_dtype, rows, w->rows, w->inner))) return st;
         joined = joined && w->order == SPLOSH_Q4_TILED128 && aligned(w->packed, 16) &&
                  splosh::mma_fits(rows, w->rows, w->inner, w->row_stride_words, lda);
+        wide = wide && w->order == SPLOSH_Q4_TILED128 && aligned(w->packed, 16) && aligned(outs[i], 16) &&
+               splosh::prefill_fits(rows, w->rows, w->inner, lda, ldcs[i]);
         columns += w->rows;
+    }
+    // More than 64 rows of tiled weights: 65..128 as two grouped calls of at most 64 (as a single weight's),
+    // more as one call of the prefill kernel over the weights side by side (2048 rows of K5120 -> N5120,
+    // N1024, N1024: 225 us as three calls, 145 as one).
+    if (wide && rows > 64 && rows <= 128) {
+        const size_t esize = out_dtype == SPLOSH_F32 ? 4 : 2;
+        void *rest[SPLOSH_MAX_GROUP];
+        for (int i = 0; i < count; ++i) rest[i] = (char *)outs[i] + 64 * ldcs[i] * esize;
+        if ((st = splosh_q4_gemm_group(weights, count, a, lda, outs, ldcs, out_dtype, 64, kernel, workspace,
+                                       workspace_bytes, stream)))
+            return st;
+        return splosh_q4_gemm_group(weights, count, a + 64 * lda, lda, rest, ldcs, out_dtype, rows - 64, kernel,
+                                    workspace, workspace_bytes, stream);
+    }
+    if (wide && rows > 128 && splosh::prefill_fits(rows, columns, weights[0].inner, lda, 0)) {
+        const splosh::PrefillPlan plan =
+            splosh::plan_prefill(rows, columns, weights[0].inner / kGroupSize, workspace ? workspace_bytes : 0);
+        return hip_status(splosh::launch_q4_prefill_group(plan, weights, count, outs, ldcs, a, lda, out_dtype, rows,
+                                                          workspace, stream),
+                          "q4 grouped prefill launch");
     }
     joined = joined && splosh::mma_fits(rows, columns, weights[0].inner, 0, lda) &&
              columns * (weights[0].inner / kGroupSize) * 32 < ((int64_t)1 << 32) - 256;
@@ -683,7 +711,8 @@ static int gguf_gemm(const splosh_q5k_weight *w_in, bool fifth, const uint16_t *
                             "prefill kernel needs K % 256 == 0, N % 128 == 0, lda % 8 == 0, ldc % 4 == 0 and 16-byte "
                             "aligned operands");
             const splosh::PrefillPlan plan =
-                splosh::plan_prefill(rows, w->rows, w->inner / kGroupSize, workspace ? workspace_bytes : 0);
+                splosh::plan_prefill(rows, w->rows, w->inner / kGroupSize, workspace ? workspace_bytes : 0,
+                                     splosh::kPrefillDecodePlanes);
             return hip_status(splosh::launch_q5k_prefill(plan, *w, fifth, a, lda, out, ldc, out_dtype, residual, rows,
                                                          workspace, stream),
                               "q5k prefill launch");
@@ -847,7 +876,8 @@ static int gguf_native_gemm(int gguf_type, const uint8_t *native, int64_t rows, 
         if (workspace_bytes == 0) workspace = nullptr;
     }
     if (prefill) {
-        const splosh::PrefillPlan plan = splosh::plan_prefill(m, rows, inner / kGroupSize, workspace ? workspace_bytes : 0);
+        const splosh::PrefillPlan plan = splosh::plan_prefill(m, rows, inner / kGroupSize, workspace ? workspace_bytes : 0,
+                                                              splosh::kPrefillDecodeNative);
         return hip_status(splosh::launch_gguf_prefill(plan, gguf_type, native, rows, inner, a, lda, out, ldc, out_dtype,
                                                       residual, m, workspace, stream),
                           "gguf prefill launch");

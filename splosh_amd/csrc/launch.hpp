@@ -197,19 +197,37 @@ hipError_t launch_q4_tile(const TilePlan &plan, const splosh_q4_weight &w, const
 // The prefill kernel for one tiled weight (prefill.hip): 256 x 256 tiles, two waves per SIMD,
 // weights dequantized once a workgroup into LDS; stream-K over a caller workspace of prefill_workspace_bytes().
 struct PrefillPlan {
-    int mblocks;       // row blocks of 256
+    int fm;            // tile rows / 64 (2, 3 or 4)
+    int mblocks;       // row blocks of 64 fm
     int tiles;
     int grid;
+    int sk_grid;       // workgroups that share the other tiles
     int dp_tiles;      // tiles computed whole (a multiple of grid)
-    int64_t sk_units;  // (tile, group) pairs of the other tiles, split evenly over the grid
+    int64_t sk_units;  // (tile, group) pairs of the other tiles, split evenly over sk_grid
+};
+// The weights of a grouped call side by side (columns col[i] .. col[i + 1] - 1 are weight i's).
+struct PrefillGroup {
+    int count;
+    int col[SPLOSH_MAX_GROUP + 1];
+    const void *w[SPLOSH_MAX_GROUP][3];
+    void *out[SPLOSH_MAX_GROUP];
+    int64_t ldc[SPLOSH_MAX_GROUP];
 };
 bool prefill_fits(int64_t rows, int64_t columns, int64_t inner, int64_t lda, int64_t ldc);
-PrefillPlan plan_prefill(int64_t rows, int64_t columns, int64_t groups, size_t workspace_bytes);
+// `decode`: what the format adds to a step's time (us; measured at 256-row tiles: Q4_K and Q5_K 2.1 us a
+// step against 1.75, the native formats 2.4 to 3.2).
+constexpr double kPrefillDecodeQ4 = 0.0, kPrefillDecodePlanes = 0.35, kPrefillDecodeNative = 1.0;
+PrefillPlan plan_prefill(int64_t rows, int64_t columns, int64_t groups, size_t workspace_bytes,
+                         double decode = kPrefillDecodeQ4);
 size_t prefill_workspace_bytes(int64_t rows, int64_t columns, int64_t groups);
 // emit: null, or the operand to write from the epilogue (fp32 output, n % 64 == 0).
 hipError_t launch_q4_prefill(const PrefillPlan &plan, const splosh_q4_weight &w, const uint16_t *a, int64_t lda,
                              void *out, int64_t ldc, int out_dtype, const void *residual, int64_t rows,
                              void *workspace, hipStream_t stream, const EmitOperand *emit = nullptr);
+// Several tiled weights of one inner size on one activation (plan: the sum of their columns).
+hipError_t launch_q4_prefill_group(const PrefillPlan &plan, const splosh_q4_weight *w, int count, void *const *outs,
+                                   const int64_t *ldcs, const uint16_t *a, int64_t lda, int out_dtype, int64_t rows,
+                                   void *workspace, hipStream_t stream);
 // Fused gate+up (silu(g) * u) over two TILED128 weights of one geometry: tiles of 128 columns of
 // each; plan with plan_prefill(rows, 2 * columns, groups, ...).
 hipError_t launch_q4_prefill_mlp(const PrefillPlan &plan, const splosh_q4_weight &gate, const splosh_q4_weight &up,

@@ -1,10 +1,11 @@
 // prefill.hip -- q4 GEMM for prefill (hundreds to thousands of activation rows) on
 // v_mfma_f32_32x32x16_bf16, two waves per SIMD.
 //
-// A workgroup of eight waves computes a 256 x 256 output tile; wave (wm, wn) = (wave / 4,
-// wave % 4) owns rows 128 wm .. 128 wm + 127 of columns 64 wn .. 64 wn + 63 (4 x 2 MFMA tiles of
-// 32 x 32: 128 fp32 accumulators a lane, in AGPRs). Per 64-group of K:
-//  * the activations A[256][64] go straight into LDS (buffer loads with the LDS modifier), rows of
+// A workgroup of eight waves computes an output tile of 64 FM rows (FM = 4, 3 or 2: 256, 192 or 128,
+// whichever plan_prefill expects the call to be fastest with) by 256 columns; wave (wm, wn) =
+// (wave / 4, wave % 4) owns rows 32 FM wm .. + 32 FM - 1 of columns 64 wn .. + 63 (FM x 2 MFMA tiles of
+// 32 x 32: 32 FM fp32 accumulators a lane, in AGPRs). Per 64-group of K:
+//  * the activations A[64 FM][64] go straight into LDS (buffer loads with the LDS modifier), rows of
 //    128 bytes whose 16-byte pieces are swizzled: piece P of row R sits at slot P ^ ((R / 2) mod 8),
 //    so that a wave's writes are contiguous and the operand reads of 16 consecutive rows hit 16
 //    different bank groups;
@@ -21,9 +22,9 @@
 //
 // Work split. Tiles are numbered row block first (tile t: row block t mod MB, column block t / MB),
 // so that with eight row blocks every XCD (workgroup id mod 8) works on one row block and keeps
-// its activations in its L2. As in mma.hip, whole tiles go round-robin over the grid and the
-// remaining tiles' (tile, group) pairs are split evenly over all workgroups (stream-K); a tile
-// covered in part is summed by prefill_finish from fp32 partials in the caller's workspace.
+// its activations in its L2. Whole tiles go round-robin over the grid; the remaining
+// tiles are whole too, or their (tile, group) pairs are split evenly over sk_grid workgroups
+// (plan_prefill); a tile covered in part is summed by prefill_finish from fp32 partials in the caller's workspace.
 //
 // Numerics as mma.hip: fp32 dequantized weight rounded to bf16, exact products, fp32 sums.
 #include "common.hpp"
@@ -50,15 +51,30 @@ struct PrefillArgs {
     const void *residual;
     int64_t rows;
     int out_dtype;
-    int mblocks;        // row blocks of 256
-    float *partial;     // stream-K partial tiles [gridDim.x][2][256][256]
+    int mblocks;        // row blocks of 64 FM
+    float *partial;     // stream-K partial tiles [sk_grid][2][64 FM][256]
     int dp_tiles;       // tiles computed whole (a multiple of gridDim.x)
-    int64_t sk_units;   // (tile, group) pairs of the remaining tiles
+    int64_t sk_units;   // (tile, group) pairs of the remaining tiles, split evenly over sk_grid workgroups
+    int sk_grid;
     uint32_t a_bytes;
     // The next RMSNorm's operand, written from the epilogue (one weight, fp32 output, N % 64 == 0;
     // null norm_weight: none).
     EmitOperand emit;
+    PrefillGroup group; // a grouped call (Q4GroupStage): the weights and outputs by column
 };
+
+// Where column n of a call's outputs goes: index m ldc + n from `out` (of a grouped call: the weight that
+// owns n, its output moved back by the weight's first column).
+struct PrefillTarget {
+    void *out;
+    int64_t ldc;
+};
+__device__ __forceinline__ PrefillTarget prefill_target(const PrefillGroup &g, int64_t n, int out_dtype) {
+    int gi = 0;
+    for (int i = 1; i < g.count; ++i) gi = n >= g.col[i] ? i : gi;
+    const int64_t back = g.col[gi] * (out_dtype == SPLOSH_F32 ? 4 : 2);
+    return PrefillTarget{(char *)g.out[gi] - back, g.ldc[gi]};
+}
 
 constexpr int kPB = 256;                       // tile rows and columns
 constexpr int kPRow = 144;                     // LDS bytes per weight column (128 + 16)
@@ -130,7 +146,8 @@ __device__ __forceinline__ void prefill_emit_band(const EmitOperand &e, int64_t 
 // workgroup's partial tile `slot`.
 template <int FM, bool EMIT>
 __device__ __forceinline__ void prefill_store_tile(const PrefillArgs &args, const f32x16 (&acc)[FM][2], char *epi,
-                                                   int64_t m0, int64_t ncol, int tc0, int tr0, int lane, int slot) {
+                                                   int64_t m0, int64_t ncol, int tc0, int tr0, int lane, int slot,
+                                                   PrefillTarget to) {
     const int r = lane & 31, h = lane >> 5;
 #pragma unroll
     for (int f = 0; f < FM; ++f) {
@@ -149,17 +166,18 @@ __device__ __forceinline__ void prefill_store_tile(const PrefillArgs &args, cons
             const int64_t m = m0 + tr + row, n = ncol + c4;
             const bool live = m < args.rows && n < args.n;
             if (EMIT && slot < 0 && args.emit.norm_weight) {  // fp32 output, whole 64-column bands
-                const f32x4 h = live ? prefill_out4(args.out, args.ldc, SPLOSH_F32, args.residual, m, n, v) : v;
+                const f32x4 h = live ? prefill_out4(to.out, to.ldc, SPLOSH_F32, args.residual, m, n, v) : v;
                 prefill_emit_band(args.emit, args.n, m, n, h, live, lane);
                 continue;
             }
             if (!live) continue;
             if (slot >= 0) {
-                float *dst = args.partial + ((int64_t)(blockIdx.x * 2 + slot) * kPB + tr + row) * kPB + tc0 + c4;
+                float *dst =
+                    args.partial + ((int64_t)(blockIdx.x * 2 + slot) * (64 * FM) + tr + row) * kPB + tc0 + c4;
                 *(f32x4 *)dst = v;
                 continue;
             }
-            prefill_out4(args.out, args.ldc, args.out_dtype, args.residual, m, n, v);
+            prefill_out4(to.out, to.ldc, args.out_dtype, args.residual, m, n, v);
         }
     }
 }
@@ -218,6 +236,7 @@ __device__ __forceinline__ void prefill_store_mlp(const PrefillArgs &args, const
 // and the column's scale and bias (Retile.swift:135-153), dequantized by dequant_word_fp8.
 struct Q4Stage {
     static constexpr int kLoads = 3, kNW = 1;
+    static constexpr bool kGrouped = false;
     static constexpr bool kEmit = true;  // the epilogue can write the next norm's operand
     rsrc_t q_rsrc, s_rsrc, b_rsrc;
     uint32_t c_src, s_src;
@@ -251,9 +270,28 @@ struct Q4Stage {
 // 0 .. 255) and the same 128 of the up weight (threads 256 .. 511).
 struct Q4PairStage : Q4Stage {
     static constexpr int kNW = 2;
+    static constexpr bool kGrouped = false;
     static constexpr bool kEmit = false;
     __device__ Q4PairStage(const PrefillArgs &args)
         : Q4Stage(args, __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) != 0) {}
+};
+
+// Several tiled q4 weights side by side (a grouped call): the tile's columns run over the weights in
+// order. A weight is whole 128-column tiles, so a wave's 32 columns lie in one.
+struct Q4GroupStage : Q4Stage {
+    static constexpr bool kEmit = false, kGrouped = true;
+    __device__ Q4GroupStage(const PrefillArgs &args) : Q4Stage(args) {}
+    __device__ void begin(const PrefillArgs &args, uint32_t col, int hh) {
+        const PrefillGroup &g = args.group;
+        const int first = __builtin_amdgcn_readfirstlane((int)col);
+        int gi = 0;
+        for (int i = 1; i < g.count; ++i) gi = first >= g.col[i] ? i : gi;
+        const uint32_t recs = (uint32_t)(g.col[gi + 1] - g.col[gi]) * (uint32_t)args.groups;
+        q_rsrc = make_rsrc(g.w[gi][0], recs * 32u);
+        s_rsrc = make_rsrc(g.w[gi][1], recs * 2u);
+        b_rsrc = make_rsrc(g.w[gi][2], recs * 2u);
+        Q4Stage::begin(args, col - (uint32_t)g.col[gi], hh);
+    }
 };
 
 // GGUF Q5_K / Q4_K planes (GgufPlanes.swift:8-20, 62-74): the thread's 32-element group j of its
@@ -270,6 +308,7 @@ struct Q4PairStage : Q4Stage {
 template <bool FIFTH>
 struct Q5Stage {
     static constexpr int kLoads = FIFTH ? 3 : 2, kNW = 1;
+    static constexpr bool kGrouped = false;
     static constexpr bool kEmit = false;
     rsrc_t p0_rsrc, p1_rsrc, m_rsrc;
     uint32_t p0_src, p1_src, m_src;
@@ -348,6 +387,7 @@ struct Q5Stage {
 template <int TYPE>
 struct GgufStage {
     static constexpr int kLoads = 0, kNW = 1;
+    static constexpr bool kGrouped = false;
     static constexpr bool kEmit = false;
     rsrc_t r;
     GgufRow row;
@@ -377,19 +417,19 @@ struct GgufStage {
 };
 
 // The kernel's buffers (see the top of the file).
-constexpr int kSA = kPB * 128;                 // swizzled activations of a group
-constexpr int kSBuf = kSA + kPABuf;            // activations and bf16 weights of a group
-constexpr size_t kSLds = 2 * (size_t)kSBuf;
-constexpr int kSALoads = 4;                    // activation loads (into LDS) of a wave and group
-static_assert(8 * kPEpi <= (int)kSLds, "eight waves' epilogue staging fits the buffers");
+// (64 FM rows.)
+constexpr int prefill_a_bytes(int fm) { return 64 * fm * 128; }
+constexpr int prefill_buf(int fm) { return prefill_a_bytes(fm) + kPABuf; }  // activations and bf16 weights of a group
+constexpr size_t prefill_lds(int fm) { return 2 * (size_t)prefill_buf(fm); }
+static_assert(8 * kPEpi <= (int)prefill_lds(2), "eight waves' epilogue staging fits the buffers");
 
-template <class W>
-__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
-prefill_kernel(PrefillArgs args) {
+template <class W, int FM>
+__device__ __forceinline__ void prefill_body(const PrefillArgs &args) {
     constexpr int kSCodeLoads = W::kLoads;
     constexpr int NW = W::kNW;          // 2: fused gate+up, 128 columns of each weight a tile
     constexpr int kTileCols = kPB / NW; // output columns a tile
-    constexpr int FM = 4, kAPer = 4;
+    constexpr int kAPer = FM;           // activation loads (into LDS) of a wave and group
+    constexpr int kSA = prefill_a_bytes(FM), kSBuf = prefill_buf(FM);
     extern __shared__ __align__(16) char lds[];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -413,7 +453,7 @@ prefill_kernel(PrefillArgs args) {
 
     auto run_job = [&](int tile, int ga, int gb, int slot) {
         const int mb = tile % args.mblocks, nb = tile / args.mblocks;
-        const int64_t m0 = (int64_t)mb * kPB, n0 = (int64_t)nb * kTileCols;
+        const int64_t m0 = (int64_t)mb * (64 * FM), n0 = (int64_t)nb * kTileCols;
         const int T = gb - ga;
         // Activation load p of this wave writes LDS bytes [8192 p + 1024 wave, + 1024): lane l takes
         // row 64 p + 8 wave + l / 8, slot l % 8, i.e. piece (l % 8) ^ ((row / 2) mod 8) (rows past
@@ -453,7 +493,7 @@ prefill_kernel(PrefillArgs args) {
         };
         // Operands of MFMA step i (k = 32 h + 8 i .. + 7 of the group, piece 4 h + i of a row).
         auto read_ops = [&](bf16x8 *af, bf16x8 *bw, int buf, int i) {
-            const char *pa = lds + buf * kSBuf + (128 * wm + r) * 128 + (((4 * h + i) ^ swz) << 4);
+            const char *pa = lds + buf * kSBuf + (32 * FM * wm + r) * 128 + (((4 * h + i) ^ swz) << 4);
 #pragma unroll
             for (int f = 0; f < FM; ++f) af[f] = as_bf16x8(*(const u32x4 *)(pa + f * 32 * 128));
             const char *pb = lds + buf * kSBuf + kSA + (64 * wn + r) * kPRow + (4 * h + i) * 16;
@@ -517,13 +557,16 @@ prefill_kernel(PrefillArgs args) {
         if (NW == 2 && slot < 0)
             prefill_store_mlp<FM>(args, acc, lds, wave, m0, ncol, 32 * FM * wm, lane);
         else
-            prefill_store_tile<FM, W::kEmit>(args, acc, epi, m0, ncol, 64 * wn, 32 * FM * wm, lane, slot);
+            prefill_store_tile<FM, W::kEmit>(args, acc, epi, m0, ncol, 64 * wn, 32 * FM * wm, lane, slot,
+                                             W::kGrouped ? prefill_target(args.group, ncol, args.out_dtype)
+                                                         : PrefillTarget{args.out, args.ldc});
     };
 
     const int P = gridDim.x;
     int dp_tile = blockIdx.x;
-    int64_t u = args.sk_units * blockIdx.x / P;
-    const int64_t u_end = args.sk_units * (blockIdx.x + 1) / P;
+    const bool shares = (int)blockIdx.x < args.sk_grid;
+    int64_t u = shares ? args.sk_units * blockIdx.x / args.sk_grid : 0;
+    const int64_t u_end = shares ? args.sk_units * (blockIdx.x + 1) / args.sk_grid : 0;
     int slot = 0;
     for (;;) {
         int tile, ga, gb, job_slot;
@@ -548,13 +591,25 @@ prefill_kernel(PrefillArgs args) {
     }
 }
 
+// 256-row tiles of one weight or the fused pair; lower tiles and grouped weights.
+template <class W>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+prefill_kernel(PrefillArgs args) {
+    prefill_body<W, 4>(args);
+}
+template <class W, int FM>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+prefill_tile_kernel(PrefillArgs args) {
+    prefill_body<W, FM>(args);
+}
+
 // Sums the stream-K partials of the remainder tiles in workgroup order and applies the epilogue.
 // Block (rt, y) covers elements [1024 y, 1024 y + 1024) of remainder tile rt, four a thread; its
 // first thread lists the tile's contributing workgroups once (see q4_mma_finish).
 __global__ void __launch_bounds__(256)
 prefill_finish(const float *__restrict__ partial, int dp_tiles, int64_t sk_units, int P, int64_t groups,
-                  int mblocks, int64_t rows, int64_t n, void *out, int64_t ldc, int out_dtype, const void *residual,
-                  int nw, EmitOperand emit) {
+                  int mblocks, int tile_rows, int64_t rows, int64_t n, void *out, int64_t ldc, int out_dtype,
+               const void *residual, int nw, EmitOperand emit, PrefillGroup group) {
     __shared__ int wg[kPFinishMax];
     __shared__ int slot_of[kPFinishMax];
     __shared__ int count;
@@ -577,7 +632,7 @@ prefill_finish(const float *__restrict__ partial, int dp_tiles, int64_t sk_units
     if (contributors <= 1) return;  // one workgroup covered the tile and wrote it
     const int tile = dp_tiles + (int)rt;
     const int cols = kPB / nw;  // output columns a tile (nw = 2: gate at tc, up at tc + 128)
-    const int64_t m0 = (int64_t)(tile % mblocks) * kPB, n0 = (int64_t)(tile / mblocks) * cols;
+    const int64_t m0 = (int64_t)(tile % mblocks) * tile_rows, n0 = (int64_t)(tile / mblocks) * cols;
     const int e0 = (blockIdx.y * 256 + threadIdx.x) * 4;  // element of the tile
     const int tr = e0 / cols, tc = e0 % cols;
     const int64_t m = m0 + tr, col = n0 + tc;
@@ -590,7 +645,7 @@ prefill_finish(const float *__restrict__ partial, int dp_tiles, int64_t sk_units
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 const int jj = j0 + j < contributors ? j0 + j : contributors - 1;
-                x[j] = *(const f32x4 *)(partial + ((int64_t)(wg[jj] * 2 + slot_of[jj]) * kPB + tr) * kPB + c);
+                x[j] = *(const f32x4 *)(partial + ((int64_t)(wg[jj] * 2 + slot_of[jj]) * tile_rows + tr) * kPB + c);
             }
 #pragma unroll
             for (int j = 0; j < 8; ++j)
@@ -611,7 +666,8 @@ prefill_finish(const float *__restrict__ partial, int dp_tiles, int64_t sk_units
         prefill_emit_band(emit, n, m, col, h, live, (int)threadIdx.x & 63);
         return;
     }
-    prefill_out4(out, ldc, out_dtype, residual, m, col, v);
+    const PrefillTarget to = group.count > 0 ? prefill_target(group, col, out_dtype) : PrefillTarget{out, ldc};
+    prefill_out4(to.out, to.ldc, out_dtype, residual, m, col, v);
 }
 
 // One tiled weight, 16-byte aligned rows of activations and outputs (vector epilogue), 32-bit
@@ -636,27 +692,80 @@ static int prefill_grid() {
 // The workspace's first 16 KiB hold the other kernels' arrival counters (left at zero between
 // calls); the partial tiles follow them.
 constexpr size_t kPCounterBytes = 16384;
-static size_t prefill_sk_bytes(int grid) { return kPCounterBytes + (size_t)grid * 2 * kPB * kPB * sizeof(float); }
+static size_t prefill_sk_bytes(int grid, int fm) {
+    return kPCounterBytes + (size_t)grid * 2 * (64 * fm) * kPB * sizeof(float);
+}
 
-PrefillPlan plan_prefill(int64_t rows, int64_t columns, int64_t groups, size_t workspace_bytes) {
-    PrefillPlan p;
-    p.mblocks = (int)((rows + kPB - 1) / kPB);
-    p.tiles = p.mblocks * (int)((columns + kPB - 1) / kPB);
-    p.grid = prefill_grid();
-    p.dp_tiles = (p.tiles / p.grid) * p.grid;
-    p.sk_units = (int64_t)(p.tiles - p.dp_tiles) * groups;
-    if (p.sk_units > 0 && prefill_sk_bytes(p.grid) > workspace_bytes) {
-        // No room for partials: every tile whole, one workgroup each.
-        p.grid = p.tiles;
-        p.dp_tiles = p.tiles;
-        p.sk_units = 0;
+// How a call is cut, by an estimate of its time (us) from what the kernel measured on this part (q4,
+// K5120 and K17408, 200 to 2048 rows, every tile height and split):
+//  * a step of a tile of 128, 192 or 256 rows takes 0.87, 1.18 or 1.37 us while at most about 60% of
+//    the CUs work, and 1.12, 1.45 or 1.8 with all of them (the shader clock falls under the load, so a
+//    round that leaves CUs idle loses little: 160 whole tiles of 80 steps, K5120 -> N5120 at 2048 rows,
+//    take 119 us, split over all 256 CUs 132). `decode` is what the format's decoding adds to a step;
+//  * a call whose last tiles are split costs 8.5 us more for the finish pass's launch and the partials'
+//    round trip, and 0.15 us a megabyte of partials.
+// Whole rounds of tiles come first; the remaining tiles are left whole, cut into S slices each (S a
+// tile's workgroups, so that no workgroup meets two tiles), or split evenly over all CUs. Measured
+// against even splits of 256-row tiles (us): 333 rows K5120 -> N5120 53.9 -> 40.6 (128 rows, 4 slices),
+// N7168 63 -> 49 (192, 4), N12288 86 -> 71 (192, 2), K17408 -> N5120 104 -> 87 (192, 6), gate+up 180 ->
+// 152 (192); 1024 rows N5120 84 -> 75 (256, 3), N12288 155 -> 134 (256, whole); 2048 rows N5120 132 ->
+// 119, N7168 174 -> 145 (256, whole).
+static double prefill_step_us(int fm, double busy, double decode) {
+    static const double kIdle[5] = {0, 0, 0.87, 1.18, 1.37}, kFull[5] = {0, 0, 1.12, 1.45, 1.8};
+    const double x = busy <= 0.6 ? 0.0 : busy >= 1.0 ? 1.0 : (busy - 0.6) / 0.4;
+    return kIdle[fm] + (kFull[fm] - kIdle[fm]) * x + decode;
+}
+
+PrefillPlan plan_prefill(int64_t rows, int64_t columns, int64_t groups, size_t workspace_bytes, double decode) {
+    const int cus = prefill_grid();
+    PrefillPlan best = {};
+    double best_us = 0.0;
+    for (int fm = 4; fm >= 2; --fm) {
+        PrefillPlan p = {};
+        p.fm = fm;
+        p.mblocks = (int)((rows + 64 * fm - 1) / (64 * fm));
+        p.tiles = p.mblocks * (int)((columns + kPB - 1) / kPB);
+        const int full = p.tiles / cus * cus, rem = p.tiles - full;
+        const double tile_mb = 64.0 * fm * kPB * 4 / 1e6;
+        const double whole = full / cus * (double)groups * prefill_step_us(fm, 1.0, decode);
+        // s = 0: the remaining tiles evenly over all CUs; 1: whole; more: slices a tile.
+        for (int s = 0; s <= 16; ++s) {
+            if ((s != 1 && rem == 0) || (s > 1 && ((int64_t)rem * s > cus || s > groups))) continue;
+            p.grid = p.tiles < cus ? p.tiles : cus;
+            p.dp_tiles = p.tiles;
+            p.sk_units = 0;
+            p.sk_grid = 0;
+            double us = whole;
+            if (s == 1) {
+                if (rem > 0) us += groups * prefill_step_us(fm, (double)rem / cus, decode);
+            } else {
+                p.dp_tiles = full;
+                p.sk_units = (int64_t)rem * groups;
+                p.sk_grid = s == 0 ? cus : rem * s;
+                p.grid = full > 0 ? cus : p.sk_grid;
+                if (prefill_sk_bytes(p.sk_grid, fm) > workspace_bytes) continue;  // no room for partials
+                const double parts = p.sk_grid + (s == 0 ? rem : 0);
+                us += (double)((p.sk_units + p.sk_grid - 1) / p.sk_grid) *
+                          prefill_step_us(fm, (double)p.sk_grid / cus, decode) +
+                      8.5 + 0.15 * parts * tile_mb;
+            }
+            if (best.fm == 0 || us < best_us) {
+                best = p;
+                best_us = us;
+            }
+        }
     }
-    return p;
+    return best;
 }
 
 size_t prefill_workspace_bytes(int64_t rows, int64_t columns, int64_t groups) {
-    const PrefillPlan p = plan_prefill(rows, columns, groups, (size_t)-1);
-    return p.sk_units > 0 ? prefill_sk_bytes(p.grid) : 0;
+    size_t need = 0;
+    for (const double decode : {kPrefillDecodeQ4, kPrefillDecodePlanes, kPrefillDecodeNative}) {
+        const PrefillPlan p = plan_prefill(rows, columns, groups, (size_t)-1, decode);
+        const size_t bytes = p.sk_units > 0 ? prefill_sk_bytes(p.sk_grid, p.fm) : 0;
+        need = need > bytes ? need : bytes;
+    }
+    return need;
 }
 
 template <class W>
@@ -677,19 +786,27 @@ static hipError_t launch_prefill(const PrefillPlan &plan, PrefillArgs &args, int
     args.dp_tiles = plan.dp_tiles;
     args.sk_units = plan.sk_units;
     args.a_bytes = (uint32_t)(((rows - 1) * lda + inner) * 2);
-    static bool once = [] {
-        (void)hipFuncSetAttribute((const void *)prefill_kernel<W>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  (int)kSLds);
+    args.sk_grid = plan.sk_grid;
+    void (*high)(PrefillArgs);
+    if constexpr (W::kGrouped) high = prefill_tile_kernel<W, 4>;
+    else high = prefill_kernel<W>;
+    static const bool once = [&] {
+        (void)hipFuncSetAttribute((const void *)prefill_tile_kernel<W, 2>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)prefill_lds(2));
+        (void)hipFuncSetAttribute((const void *)prefill_tile_kernel<W, 3>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)prefill_lds(3));
+        (void)hipFuncSetAttribute((const void *)high, hipFuncAttributeMaxDynamicSharedMemorySize, (int)prefill_lds(4));
         return true;
     }();
     (void)once;
-    hipLaunchKernelGGL(prefill_kernel<W>, dim3((unsigned)plan.grid), dim3(512), kSLds, stream, args);
+    const auto kernel = plan.fm == 2 ? prefill_tile_kernel<W, 2> : plan.fm == 3 ? prefill_tile_kernel<W, 3> : high;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)plan.grid), dim3(512), prefill_lds(plan.fm), stream, args);
     hipError_t err = hipGetLastError();
     if (err != hipSuccess || plan.sk_units == 0) return err;
     const int remainder = plan.tiles - plan.dp_tiles;
-    hipLaunchKernelGGL(prefill_finish, dim3((unsigned)remainder, kPB * kPB / 1024 / W::kNW), dim3(256), 0, stream,
-                       (const float *)args.partial, plan.dp_tiles, plan.sk_units, plan.grid, args.groups, plan.mblocks,
-                       rows, n, out, ldc, out_dtype, residual, W::kNW, args.emit);
+    hipLaunchKernelGGL(prefill_finish, dim3((unsigned)remainder, 64 * plan.fm * kPB / 1024 / W::kNW), dim3(256), 0,
+                       stream, (const float *)args.partial, plan.dp_tiles, plan.sk_units, plan.sk_grid, args.groups,
+                       plan.mblocks, 64 * plan.fm, rows, n, out, ldc, out_dtype, residual, W::kNW, args.emit, args.group);
     return hipGetLastError();
 }
 
@@ -706,6 +823,33 @@ hipError_t launch_q4_prefill(const PrefillPlan &plan, const splosh_q4_weight &w,
     args.w_bytes[1] = args.w_bytes[2] = (uint32_t)(w.rows * groups * 2);
     return launch_prefill<Q4Stage>(plan, args, w.rows, w.inner, a, lda, out, ldc, out_dtype, residual, rows,
                                    workspace, stream);
+}
+
+hipError_t launch_q4_prefill_group(const PrefillPlan &plan, const splosh_q4_weight *w, int count, void *const *outs,
+                                   const int64_t *ldcs, const uint16_t *a, int64_t lda, int out_dtype, int64_t rows,
+                                   void *workspace, hipStream_t stream) {
+    PrefillArgs args = {};
+    const int64_t groups = w[0].inner / kGroup;
+    args.group.count = count;
+    int64_t columns = 0;
+    for (int i = 0; i < count; ++i) {
+        args.group.col[i] = (int)columns;
+        args.group.w[i][0] = w[i].packed;
+        args.group.w[i][1] = w[i].scales;
+        args.group.w[i][2] = w[i].biases;
+        args.group.out[i] = outs[i];
+        args.group.ldc[i] = ldcs[i];
+        columns += w[i].rows;
+    }
+    args.group.col[count] = (int)columns;
+    // The first weight's pointers stand in for the single-weight fields (never read).
+    args.w[0] = w[0].packed;
+    args.w[1] = w[0].scales;
+    args.w[2] = w[0].biases;
+    args.w_bytes[0] = (uint32_t)(w[0].rows * groups * 32);
+    args.w_bytes[1] = args.w_bytes[2] = (uint32_t)(w[0].rows * groups * 2);
+    return launch_prefill<Q4GroupStage>(plan, args, columns, w[0].inner, a, lda, outs[0], ldcs[0], out_dtype, nullptr,
+                                        rows, workspace, stream);
 }
 
 hipError_t launch_q4_prefill_mlp(const PrefillPlan &plan, const splosh_q4_weight &gate, const splosh_q4_weight &up,
