@@ -151,6 +151,10 @@ int splosh_q4_shape_validate(int64_t rows, int64_t columns, int64_t inner, const
  * as it is (zero it again after a call that failed or was aborted). */
 size_t splosh_workspace_bytes(int64_t rows, int64_t columns, int64_t inner);
 
+/* The scratch splosh_q4_gemm (pair: splosh_q4_mlp_in) can use on this weight under AUTO with
+ * activation rows lda apart: splosh_workspace_bytes at most, 0 where its kernel splits nothing. */
+size_t splosh_q4_workspace_bytes(const splosh_q4_weight *w, int64_t lda, int64_t rows, int pair);
+
 const char *splosh_status_string(int status);
 /* The message of the last failure on this thread ("" after success). */
 const char *splosh_last_error(void);

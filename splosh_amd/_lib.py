@@ -74,6 +74,7 @@ SIGNATURES = {
     "splosh_q4_layout_sidecar_index": (_int, [ctypes.POINTER(Layout), _i64, _i64, ctypes.POINTER(_i64)]),
     "splosh_q4_shape_validate": (_int, [_i64, _i64, _i64, ctypes.POINTER(Layout)]),
     "splosh_workspace_bytes": (_sz, [_i64, _i64, _i64]),
+    "splosh_q4_workspace_bytes": (_sz, [ctypes.POINTER(Q4Weight), _i64, _i64, _int]),
     "splosh_status_string": (ctypes.c_char_p, [_int]),
     "splosh_last_error": (ctypes.c_char_p, []),
     "splosh_version": (ctypes.c_char_p, []),

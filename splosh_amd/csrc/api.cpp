@@ -428,6 +428,20 @@ size_t splosh_workspace_bytes(int64_t rows, int64_t columns, int64_t inner) {
     return need > gguf ? need : gguf;
 }
 
+// The routes of q4_gemm_impl under AUTO that need less than splosh_workspace_bytes.
+size_t splosh_q4_workspace_bytes(const splosh_q4_weight *w, int64_t lda, int64_t rows, int pair) {
+    if (!w || rows <= 0 || w->rows <= 0 || w->inner < kGroupSize) return 0;
+    if (w->order == SPLOSH_Q4_TILED128) {
+        if (rows <= 2 && splosh::decode_fits(rows, w->rows, w->inner, w->order))
+            return splosh::decode_workspace_bytes(rows, w->rows, w->inner, pair ? 2 : 1);
+        if (splosh::skinny_fits(rows, w->rows, w->inner, lda, pair != 0))
+            return splosh::skinny_workspace_bytes(rows, w->rows, w->inner, pair ? 2 : 1);
+    } else if (!pair && splosh::rows_fit(rows, w->rows, w->inner, lda)) {
+        return 0;
+    }
+    return splosh_workspace_bytes(rows, w->rows, w->inner);
+}
+
 // Q4GemmRuntime.dispatch (Runtime/Q4Runtime.swift:94-145).
 int splosh_gemm_q4(const uint16_t *a, const uint32_t *packed, const uint16_t *scales, const uint16_t *biases,
                    float *c, int64_t rows, int64_t columns, int64_t inner, const splosh_q4_layout *layout,

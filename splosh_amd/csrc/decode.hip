@@ -300,20 +300,12 @@ q4_decode_kernel(DecodeArgs args) {
     write_rows();
 }
 
-static int decode_cus() {
-    int dev = 0, cus = 256;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-        cus = 256;
-    return cus;
-}
-
 // Row block: 32 rows when that gives at least two workgroups a CU; else 8 for long K (at least 128
 // groups), where 16-row blocks would leave a CU one or two workgroups for a long loop (K17408 ->
 // N5120: 640 blocks of 8 rows with the balance split 13.3 us, 320 of 16 rows 15.4 us); else 16
 // (K5120 -> N5120: 6.5 us at 16 rows, 7.1 at 8).
 static int decode_block(int64_t columns, int64_t groups) {
-    const int64_t cus = decode_cus();
+    const int64_t cus = device_cus();
     if (columns / 32 >= 2 * cus) return 32;
     return groups >= 128 && columns / 16 < 2 * cus ? 8 : 16;
 }
@@ -339,7 +331,7 @@ bool decode_fits(int64_t rows, int64_t columns, int64_t inner, int order) {
 }
 
 static BalanceSplit plan_decode_split(int64_t columns, int groups) {
-    return plan_balance(columns / decode_block(columns, groups), decode_cus(), groups);
+    return plan_balance(columns / decode_block(columns, groups), device_cus(), groups);
 }
 
 size_t decode_workspace_bytes(int64_t rows, int64_t columns, int64_t inner, int nw) {
@@ -369,7 +361,7 @@ static hipError_t launch_decode_v(const DecodeArgs &args, hipStream_t stream) {
         decode_lds_attribute<R, NW, B, kDecodeDeepDepth>();
     }
     const unsigned grid = args.slices > 1 ? (unsigned)(args.nwhole + args.tail * args.slices) : (unsigned)(args.n / B);
-    if (NW == 1 && args.n / B <= (int64_t)kDecodeDeepBlocksPerCu * decode_cus())
+    if (NW == 1 && args.n / B <= (int64_t)kDecodeDeepBlocksPerCu * device_cus())
         hipLaunchKernelGGL((q4_decode_kernel<R, NW, B, kDecodeDeepDepth>), dim3(grid), dim3(kDecodeWg), lds, stream,
                            args);
     else

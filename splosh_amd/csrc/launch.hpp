@@ -9,6 +9,9 @@
 
 namespace splosh {
 
+// Compute units of the current device (256 where it cannot be asked), looked up once a device.
+int device_cus();
+
 // Kernel-shape choice of the streaming kernels.
 struct StreamPlan {
     int mb;        // 16-row blocks per workgroup (1, 2 or 4)

@@ -33,6 +33,7 @@
 #include "launch.hpp"
 #include "mix.hpp"
 
+#include <atomic>
 #include <cstdlib>
 #include <type_traits>
 // Weight codes are read once: non-temporal loads (gfx94x cache policy nt).
@@ -1229,17 +1230,16 @@ bool q5k_mma_fits(int64_t rows, int64_t columns, int64_t inner, int64_t lda) {
            columns * (inner / 32) * 16 < limit;
 }
 
-// Compute units of the current device (the stream-K grid), cached per device.
-static int device_cus() {
-    static int cache[64] = {0};
+int device_cus() {
+    static std::atomic<int> cache[64];
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-    if (!cache[dev]) {
-        int cus = 0;
+    int cus = cache[dev].load(std::memory_order_relaxed);
+    if (cus == 0) {
         if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
-        cache[dev] = cus;
+        cache[dev].store(cus, std::memory_order_relaxed);
     }
-    return cache[dev];
+    return cus;
 }
 
 // Workspace: a fixed region of arrival counters (one per shared band, zero between calls) at the

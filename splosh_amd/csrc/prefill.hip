@@ -679,10 +679,7 @@ bool prefill_fits(int64_t rows, int64_t columns, int64_t inner, int64_t lda, int
 }
 
 static int prefill_grid() {
-    int dev = 0, cus = 256;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-        cus = 256;
+    int cus = device_cus();
     // A development override of the grid, read from the environment once per process.
     static const int grid_override = [] { const char *e = getenv("SPLOSH_PREFILL_GRID"); return e ? atoi(e) : 0; }();
     if (grid_override > 0) cus = grid_override;

@@ -245,24 +245,16 @@ bool q5k_decode_fits(int64_t rows, int64_t columns, int64_t inner) {
            columns * (inner / 32) * 16 < ((int64_t)1 << 32) - 4096;
 }
 
-static int q5k_decode_cus() {
-    int dev = 0, cus = 256;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-        cus = 256;
-    return cus;
-}
-
 // Row block: the largest of 32, 16 and 8 that gives at least two workgroups a CU.
 static int q5k_decode_block(int64_t columns) {
-    const int64_t cus = q5k_decode_cus();
+    const int64_t cus = device_cus();
     return columns / 32 >= 2 * cus ? 32 : columns / 16 >= 2 * cus ? 16 : 8;
 }
 
 size_t q5k_decode_workspace_bytes(int64_t rows, int64_t columns, int64_t inner) {
     if (rows != 1 || columns % 128 != 0 || inner % 256 != 0) return 0;
     const int block = q5k_decode_block(columns);
-    const BalanceSplit p = plan_balance(columns / block, q5k_decode_cus(), (int)(inner / 32));
+    const BalanceSplit p = plan_balance(columns / block, device_cus(), (int)(inner / 32));
     return p.slices < 2 ? 0 : kBalanceCounterBytes + (size_t)p.tail * p.slices * block * sizeof(float);
 }
 
@@ -297,7 +289,7 @@ hipError_t launch_q5k_decode(const splosh_q5k_weight &w, const uint16_t *a, void
     const size_t need = q5k_decode_workspace_bytes(1, w.rows, w.inner);
     args.slices = 1;
     if (need > 0 && workspace && workspace_bytes >= need) {
-        const BalanceSplit p = plan_balance(w.rows / block, q5k_decode_cus(), args.groups);
+        const BalanceSplit p = plan_balance(w.rows / block, device_cus(), args.groups);
         args.nwhole = p.nwhole;
         args.tail = p.tail;
         args.slices = p.slices;

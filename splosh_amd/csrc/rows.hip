@@ -274,15 +274,8 @@ static bool rows_dot(int64_t rows, int64_t columns) {
 bool rows_fit(int64_t rows, int64_t columns, int64_t inner, int64_t lda) {
     if (rows < 1 || inner % kGroup != 0 || columns > (1 << 30) || inner > (1 << 30)) return false;
     if (rows_dot(rows, columns)) return true;
-    static const int cus = [] {
-        int dev = 0, n = 256;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-            n = 256;
-        return n;
-    }();
     // (The activations are read through a buffer resource: 32-bit byte offsets.)
-    return rows > 64 && (rows + 31) / 32 * ((columns + 31) / 32) <= cus &&
+    return rows > 64 && (rows + 31) / 32 * ((columns + 31) / 32) <= device_cus() &&
            (rows * lda + inner) * 2 < ((int64_t)1 << 32) - 256;
 }
 

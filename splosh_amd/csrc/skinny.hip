@@ -260,14 +260,6 @@ q4_skinny_kernel(SkinnyArgs args) {
     }
 }
 
-static int skinny_cus() {
-    int dev = 0, cus = 256;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-        cus = 256;
-    return cus;
-}
-
 static int skinny_rows(int64_t rows) { return rows <= 8 ? 8 : rows <= 16 ? 16 : 32; }
 
 // How a call is cut: KW waves a workgroup, and K slices of its blocks of 32 columns (NW weights
@@ -286,7 +278,7 @@ struct SkinnyPlan {
 };
 static SkinnyPlan plan_skinny(int64_t blocks, int groups) {
     SkinnyPlan p;
-    const int cus = skinny_cus();
+    const int cus = device_cus();
     p.kw = blocks >= 2 * cus ? 4 : 8;
     p.split = plan_balance(blocks, cus, groups);
     int s = 1;
@@ -304,7 +296,7 @@ static SkinnyPlan plan_skinny(int64_t blocks, int groups) {
 // K slices that make up for them (K17408 -> N5120, 16 rows 19.9 -> 17.5). Not between one and two a
 // CU (N17408, 272 pairs: 15.6 -> 19).
 static bool skinny_split(int64_t columns, int groups) {
-    const int64_t cus = skinny_cus(), blocks = columns / kSkinnyCols, pairs = blocks / 2;
+    const int64_t cus = device_cus(), blocks = columns / kSkinnyCols, pairs = blocks / 2;
     if (columns % 256 != 0) return false;  // the halves start on a 128-row tile
     return pairs >= 2 * cus || (blocks > cus && pairs <= cus) ||
            (blocks <= cus && 2 * blocks > cus && groups >= kSkinnyLong * 8);
@@ -319,7 +311,7 @@ bool skinny_fits(int64_t rows, int64_t columns, int64_t inner, int64_t lda, bool
     if (rows < 1 || rows > 32 || columns % 128 != 0 || inner % kGroup != 0 ||
         (rows * lda + inner) * 2 >= ((int64_t)1 << 30) || columns * (inner / kGroup) * 32 >= ((int64_t)1 << 32) - 4096)
         return false;
-    const int64_t cus = skinny_cus(), blocks = columns / kSkinnyCols;
+    const int64_t cus = device_cus(), blocks = columns / kSkinnyCols;
     return rows <= 16 || pair || (columns % 256 == 0 && blocks / 2 >= 2 * cus) ||
            (blocks <= cus && inner / kGroup < kSkinnyLong * 8);
 }

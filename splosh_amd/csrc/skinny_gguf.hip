@@ -529,20 +529,13 @@ gguf_skinny_kernel(SkinnyGgufArgs args) {
     }
 }
 
-static int sg_cus() {
-    int dev = 0, cus = 256;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-        cus = 256;
-    return cus;
-}
 // K slices of the blocks of 32 columns: the last round of many blocks (plan_balance); one workgroup a
 // CU for at most half a block a CU (K5120 -> N1024 9.8 -> 8.9 us); two a CU for fewer blocks than CUs
 // and long K (K17408 -> N5120, Q6_K 27.6 -> 25.8 us, Q8_0 30.8 -> 27.5; the merge costs about 3 us, which
 // K5120 -> N5120 does not win back: 11.1 -> 15).
 constexpr int kSgLong = 32;  // units of K
 static BalanceSplit plan_sg(int64_t blocks, int units) {
-    const int cus = sg_cus();
+    const int cus = device_cus();
     BalanceSplit p = plan_balance(blocks, cus, units);
     int s = 1;
     if (2 * blocks <= cus) s = (int)(cus / blocks) * (units >= kSgLong ? 2 : 1);

@@ -10,6 +10,7 @@ libsplosh_q4.so through its C ABI. The names follow the reference's host API:
 
 Buffer-size checks (GemmQ4Error.bufferTooSmall) happen here because the C ABI sees raw pointers.
 """
+import contextlib
 import ctypes
 from dataclasses import dataclass
 
@@ -27,6 +28,8 @@ SCALAR = _lib.KERNEL_SCALAR
 PREFILL = _lib.KERNEL_PREFILL
 ROW_MAJOR = _lib.ROW_MAJOR
 TILED128 = _lib.TILED128
+# The start of a workspace the kernels need zeroed before its first use (their arrival counters).
+WORKSPACE_COUNTER_BYTES = 16384
 
 
 def _ptr(t):
@@ -142,11 +145,16 @@ def _on(stream):
     return stream if stream is not None else torch.cuda.current_stream()
 
 
+def _allocating(stream):
+    """The context a call's own tensors are allocated in: the stream the kernel uses them from, so
+    torch's caching allocator orders any reuse of the block after that kernel. Nothing to enter when
+    that is torch's current stream already (entering it costs a small call 4 us)."""
+    return contextlib.nullcontext() if stream is None else torch.cuda.stream(stream)
+
+
 def _out(a, rows, n, out, out_dtype, stream=None):
     if out is None:
-        # Allocated on the stream the kernel writes it from, so torch's caching allocator orders
-        # any reuse of the block after that kernel.
-        with torch.cuda.stream(_on(stream)):
+        with _allocating(stream):
             out = torch.empty((rows, n), dtype=out_dtype, device=a.device)
     return out
 
@@ -219,10 +227,14 @@ class _Scratch:
         return iter((self.ptr, self.nbytes))
 
 
-def _workspace(workspace, rows, n, inner, device, stream=None, heads=False):
+def _workspace(workspace, rows, n, inner, device, stream=None, heads=False, q4=None):
     """The split-K scratch of the kernels: the caller's tensor (an empty one: none), or a fresh one
-    from torch's stream-ordered allocator sized by splosh_workspace_bytes. A fresh one is
-    zero-filled and allocated on the stream the kernel runs on, so the fill is ordered before the
+    from torch's stream-ordered allocator sized by splosh_workspace_bytes, or, for a q4 call under
+    AUTO (``q4``: the weight, the row stride and the pair flag), by splosh_q4_workspace_bytes: a
+    5 MB fill that the one-row kernels never look at, and entering the current stream twice, were
+    two thirds of the smallest eager call (K5120 -> N1024, one row 35.4 -> 12.8 us with both gone).
+    The counters of a fresh one are zeroed; it is allocated on the stream the kernel runs on, so
+    the fill is ordered before the
     kernel; the caller keeps the returned object (and with it the tensor) until the kernel has
     been launched, after which the allocator hands the block out again only to work ordered after
     that kernel on the same stream."""
@@ -230,11 +242,16 @@ def _workspace(workspace, rows, n, inner, device, stream=None, heads=False):
         return _Scratch(None, 0)
     if workspace is not None:
         return _Scratch(_ptr(workspace), workspace.numel() * workspace.element_size(), workspace)
-    need = (_lib.lib().splosh_heads_workspace_bytes if heads else _lib.lib().splosh_workspace_bytes)(rows, n, inner)
+    if q4 is not None:
+        weight, lda, pair = q4
+        need = _lib.lib().splosh_q4_workspace_bytes(ctypes.byref(weight), lda, rows, pair)
+    else:
+        need = (_lib.lib().splosh_heads_workspace_bytes if heads else _lib.lib().splosh_workspace_bytes)(rows, n, inner)
     if need == 0:
         return _Scratch(None, 0)
-    with torch.cuda.stream(_on(stream)):
-        buf = torch.zeros(need, dtype=torch.uint8, device=device)
+    with _allocating(stream):
+        buf = torch.empty(need, dtype=torch.uint8, device=device)
+        buf[:WORKSPACE_COUNTER_BYTES].zero_()
     return _Scratch(_ptr(buf), need, buf)
 
 
@@ -259,9 +276,12 @@ def gemm(w, a, out=None, residual=None, out_dtype=torch.bfloat16, kernel=AUTO, r
             raise SploshError(13, "residual must match the output's dtype and row stride")
     if key_heads and isinstance(w, Q4Weight):
         raise SploshError(13, "the value-head order applies to GGUF weights only")
-    scratch = _workspace(workspace, rows, w.rows, w.inner, a.device, stream, heads=bool(key_heads))  # held until the launch
-    ws, ws_bytes = scratch
-    if isinstance(w, GgufWeight):
+    is_q4 = isinstance(w, Q4Weight)
+    wc = None if isinstance(w, GgufWeight) else w.c()
+    scratch = _workspace(workspace, rows, w.rows, w.inner, a.device, stream, heads=bool(key_heads),
+                         q4=(wc, a.stride(0), 0) if is_q4 and kernel == AUTO else None)
+    ws, ws_bytes = scratch  # (scratch is held until the launch)
+    if wc is None:
         if key_heads:
             st = _lib.lib().splosh_gguf_gemm_heads(w.type_id, _ptr(w.native), w.rows, w.inner, key_heads, _ptr(a),
                                                    a.stride(0), _ptr(out), out.stride(0), _dtype_code(out.dtype),
@@ -272,13 +292,12 @@ def gemm(w, a, out=None, residual=None, out_dtype=torch.bfloat16, kernel=AUTO, r
                                              rows, ws, ws_bytes, _stream(stream))
         _lib.check(st)
         return out
-    wc = w.c()
     if key_heads:
         fn = _lib.lib().splosh_q4k_gemm_heads if isinstance(w, Q4KWeight) else _lib.lib().splosh_q5k_gemm_heads
         _lib.check(fn(ctypes.byref(wc), key_heads, _ptr(a), a.stride(0), _ptr(out), out.stride(0),
                       _dtype_code(out.dtype), _ptr(residual), rows, kernel, ws, ws_bytes, _stream(stream)))
         return out
-    if isinstance(w, Q4Weight):
+    if is_q4:
         st = _lib.lib().splosh_q4_gemm(ctypes.byref(wc), _ptr(a), a.stride(0), _ptr(out), out.stride(0),
                                        _dtype_code(out.dtype), _ptr(residual), rows, kernel, ws, ws_bytes,
                                        _stream(stream))
@@ -332,7 +351,7 @@ def gemm_emit(w, a, norm_weight, out=None, residual=None, kernel=AUTO, rows=None
     _require(out, ((rows - 1) * out.stride(0) + w.rows) * 4, "output")
     if norm_weight.dtype != torch.bfloat16 or norm_weight.numel() < w.rows:
         raise SploshError(13, "norm_weight must be bf16 with one value a column")
-    with torch.cuda.stream(_on(stream)):
+    with _allocating(stream):
         values = torch.empty((rows, w.rows), dtype=torch.bfloat16, device=a.device)
         sums = torch.empty((rows, w.rows // 64), dtype=torch.float32, device=a.device)
         squares = torch.empty_like(sums)
@@ -355,8 +374,9 @@ def mlp_in(gate, up, a, out=None, out_dtype=torch.bfloat16, kernel=AUTO, rows=No
     _require(a, ((rows - 1) * a.stride(0) + gate.inner) * 2, "a")
     _require(out, ((rows - 1) * out.stride(0) + gate.rows) * out.element_size(), "output")
     gc, uc = gate.c(), up.c()
-    scratch = _workspace(workspace, rows, gate.rows, gate.inner, a.device, stream)  # held until the launch
-    ws, ws_bytes = scratch
+    scratch = _workspace(workspace, rows, gate.rows, gate.inner, a.device, stream,
+                         q4=(gc, a.stride(0), 1) if kernel == AUTO else None)
+    ws, ws_bytes = scratch  # (scratch is held until the launch)
     st = _lib.lib().splosh_q4_mlp_in(ctypes.byref(gc), ctypes.byref(uc), _ptr(a), a.stride(0), _ptr(out),
                                      out.stride(0), _dtype_code(out.dtype), rows, kernel, ws, ws_bytes,
                                      _stream(stream))
