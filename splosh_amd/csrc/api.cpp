@@ -833,6 +833,15 @@ static int check_gguf_native(int type, const uint8_t *native, int64_t rows, int6
 }
 
 constexpr int64_t kGgufPrefillRows = 256;  // measured: the tile kernel is as fast or faster up to 128 rows
+// Rows from which weights of whole 256-element units take it instead, given the scratch of its plan: above
+// the two calls of the M <= 64 kernel (K17408 -> N5120 at 160 rows, tiled kernel and this: Q6_K 130 -> 61 us,
+// IQ3_S 160 -> 60, IQ4_XS 114 -> 56, Q8_0 125 -> 62; K1536 -> N4096 37..41 -> 23..26), and from 65 rows for the
+// weights where it wins over those: the large ones (K5120 -> N17408 at 65 and 128 rows: Q6_K 69 / 96 -> 59 / 66,
+// IQ4_XS 57 / 75 -> 51 / 57, Q8_0 65 / 80 -> 58 / 65; K11008 -> N4096 41 / 57 -> 35 / 38; but K1536 -> N11008
+// 20 / 22 -> 24 / 27 and K5120 -> N5120 26.9 / 36 -> 27.9 / 29), and Q3_K (the tiled kernel before: 84 / 87 ->
+// 49 / 55, K1536 -> N4096 24 / 24 -> 18 / 22).
+constexpr int64_t kGgufPrefillUnitRows = 129;
+constexpr int64_t kGgufPrefillLargeWeight = 40 << 20;  // elements
 
 static int gguf_native_gemm(int gguf_type, const uint8_t *native, int64_t rows, int64_t inner, const uint16_t *a,
                             int64_t lda, void *out, int64_t ldc, int out_dtype, const void *residual, int64_t m,
@@ -844,8 +853,8 @@ static int gguf_native_gemm(int gguf_type, const uint8_t *native, int64_t rows, 
         return fail(SPLOSH_ERR_UNSUPPORTED, "GGUF native kernel needs lda % 8 == 0 and 16-byte aligned activations");
     HeadOrder ho;
     if ((st = head_order(key_heads, inner, &ho))) return st;
-    // From kGgufPrefillRows rows the 256 x 256 prefill kernel (each weight group decoded once per
-    // 256 rows). Up to 64 rows the stream-K MFMA kernel (each weight group decoded once), above
+    // From kGgufPrefillRows rows (whole units: from 65 or 129) the prefill kernel (each weight group decoded
+    // once per 128 to 256 rows). Up to 64 rows the stream-K MFMA kernel (each weight group decoded once), above
     // the format's streaming limit; up to it one pass of the streaming kernel. Measured at K17408
     // -> N5120 with a workspace (us): the MFMA kernel is flat up to 32 rows (Q8_0 33, Q6_K 44, Q3_K
     // 47, IQ3_S 42, IQ4_NL 27, IQ4_XS 30); the streaming kernel at four rows Q8_0 31, Q6_K 35, Q3_K
@@ -858,14 +867,27 @@ static int gguf_native_gemm(int gguf_type, const uint8_t *native, int64_t rows, 
         const char *e = getenv("SPLOSH_GGUF_PREFILL_ROWS");
         return e ? (int64_t)atoll(e) : kGgufPrefillRows;
     }();
-    const bool prefill = m >= prefill_rows && aligned(out, 16) && (!residual || aligned(residual, 16)) &&
-                         splosh::gguf_prefill_fits(gguf_type, m, rows, inner, lda, ldc);
+    const bool units = inner % 256 == 0;
+    const double decode = units ? splosh::kPrefillDecodeUnits : splosh::kPrefillDecodeNative;
     const int base_type = gguf_type & 0xFF;
+    const int64_t from = !units ? prefill_rows
+                         : base_type == 11 || rows * inner >= kGgufPrefillLargeWeight ? 65
+                                                                                      : kGgufPrefillUnitRows;
+    bool prefill = m >= (from < prefill_rows ? from : prefill_rows) && aligned(out, 16) &&
+                   (!residual || aligned(residual, 16)) &&
+                   splosh::gguf_prefill_fits(gguf_type, m, rows, inner, lda, ldc);
+    if (prefill && m < prefill_rows) {
+        const size_t need = ho.on() ? splosh_heads_workspace_bytes(m, rows, inner)
+                                    : splosh::prefill_plan_bytes(splosh::plan_prefill(
+                                          m, rows, inner / kGroupSize, (size_t)-1, decode));
+        prefill = need == 0 || (workspace && workspace_bytes >= need);
+    }
     const int64_t stream_max = base_type == 11 ? 6 : base_type == 20 ? 3 : 4;
     // 65..128 rows: two calls of at most 64 rows, as for q4. K17408 -> N5120, against the tiled
     // kernel: M=96 Q8_0 80 -> 77 us (ROWS32 79 -> 66), Q6_K 100 -> 90, IQ3_S 105 -> 89, IQ4_NL 81 ->
-    // 63, IQ4_XS 81 -> 70; Q3_K, whose MFMA path is the slowest, 83 -> 96, keeps the tiled kernel.
-    if (base_type != 11 && m > 64 && m <= 128 && splosh::gguf_mma_fits(gguf_type, 64, rows, inner, lda)) {
+    // 63, IQ4_XS 81 -> 70; Q3_K, whose MFMA path is the slowest, 83 -> 96, keeps the tiled kernel where the
+    // prefill kernel does not take it.
+    if (!prefill && base_type != 11 && m > 64 && m <= 128 && splosh::gguf_mma_fits(gguf_type, 64, rows, inner, lda)) {
         const char *res = (const char *)residual;
         const size_t esize = out_dtype == SPLOSH_F32 ? 4 : 2;
         if ((st = gguf_native_gemm(gguf_type, native, rows, inner, a, lda, out, ldc, out_dtype, residual, 64,
@@ -891,7 +913,7 @@ static int gguf_native_gemm(int gguf_type, const uint8_t *native, int64_t rows, 
     }
     if (prefill) {
         const splosh::PrefillPlan plan = splosh::plan_prefill(m, rows, inner / kGroupSize, workspace ? workspace_bytes : 0,
-                                                              splosh::kPrefillDecodeNative);
+                                                              decode);
         return hip_status(splosh::launch_gguf_prefill(plan, gguf_type, native, rows, inner, a, lda, out, ldc, out_dtype,
                                                       residual, m, workspace, stream),
                           "gguf prefill launch");

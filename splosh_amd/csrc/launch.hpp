@@ -218,11 +218,13 @@ struct PrefillGroup {
 };
 bool prefill_fits(int64_t rows, int64_t columns, int64_t inner, int64_t lda, int64_t ldc);
 // `decode`: what the format adds to a step's time (us; measured at 256-row tiles: Q4_K and Q5_K 2.1 us a
-// step against 1.75, the native formats 2.4 to 3.2).
-constexpr double kPrefillDecodeQ4 = 0.0, kPrefillDecodePlanes = 0.35, kPrefillDecodeNative = 1.0;
+// step against 1.75, the native formats 2.0 to 2.3 in whole units of 256, else 2.4 to 3.2).
+constexpr double kPrefillDecodeQ4 = 0.0, kPrefillDecodePlanes = 0.35, kPrefillDecodeNative = 1.0, kPrefillDecodeUnits = 0.3;
 PrefillPlan plan_prefill(int64_t rows, int64_t columns, int64_t groups, size_t workspace_bytes,
                          double decode = kPrefillDecodeQ4);
 size_t prefill_workspace_bytes(int64_t rows, int64_t columns, int64_t groups);
+// The workspace a plan uses.
+size_t prefill_plan_bytes(const PrefillPlan &plan);
 // emit: null, or the operand to write from the epilogue (fp32 output, n % 64 == 0).
 hipError_t launch_q4_prefill(const PrefillPlan &plan, const splosh_q4_weight &w, const uint16_t *a, int64_t lda,
                              void *out, int64_t ldc, int out_dtype, const void *residual, int64_t rows,

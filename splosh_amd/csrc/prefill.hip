@@ -29,7 +29,7 @@
 // Numerics as mma.hip: fp32 dequantized weight rounded to bf16, exact products, fp32 sums.
 #include "common.hpp"
 #include "launch.hpp"
-#include "gguf_decode.hpp"
+#include "gguf_half.hpp"
 #include "mix.hpp"
 
 #include <cstdlib>
@@ -235,8 +235,8 @@ __device__ __forceinline__ void prefill_store_mlp(const PrefillArgs &args, const
 // MLX affine q4, TILED128: the thread's 16 bytes of the column's record (words 4 (t % 2) .. + 3)
 // and the column's scale and bias (Retile.swift:135-153), dequantized by dequant_word_fp8.
 struct Q4Stage {
-    static constexpr int kLoads = 3, kNW = 1;
-    static constexpr bool kGrouped = false;
+    static constexpr int kLoads = 3, kNW = 1, kUnit = 1, kTbl = 0;
+    static constexpr bool kGrouped = false, kTall = true;
     static constexpr bool kEmit = true;  // the epilogue can write the next norm's operand
     rsrc_t q_rsrc, s_rsrc, b_rsrc;
     uint32_t c_src, s_src;
@@ -253,13 +253,13 @@ struct Q4Stage {
         c_src = rec * 32u + 16u * hh;
         s_src = rec * 2u;
     }
-    __device__ void load(uint32_t g, int set) {
+    __device__ void load(uint32_t g, int set, int) {
         cr[set] = buffer_load16_cp<2>(q_rsrc, c_src + g * (128u * 32u), 0);
         sr[set] = buffer_load_u16(s_rsrc, s_src + g * 256u, 0);
         br[set] = buffer_load_u16(b_rsrc, s_src + g * 256u, 0);
     }
     // Words q0 and q0 + 1, pieces q0 and q0 + 1.
-    __device__ void store(char *dst, int set, uint32_t, bool on, int q0) {
+    __device__ void store(char *dst, int set, uint32_t, int, bool on, int q0) {
         const float s = on ? bf16_bits_to_f32(sr[set]) : 0.0f, b = on ? bf16_bits_to_f32(br[set]) : 0.0f;
 #pragma unroll
         for (int q = q0; q < q0 + 2; ++q) *(bf16x8 *)(dst + 16 * q) = dequant_word_fp8(cr[set][q], s, b);
@@ -279,7 +279,7 @@ struct Q4PairStage : Q4Stage {
 // Several tiled q4 weights side by side (a grouped call): the tile's columns run over the weights in
 // order. A weight is whole 128-column tiles, so a wave's 32 columns lie in one.
 struct Q4GroupStage : Q4Stage {
-    static constexpr bool kEmit = false, kGrouped = true;
+    static constexpr bool kEmit = false, kGrouped = true, kTall = false;
     __device__ Q4GroupStage(const PrefillArgs &args) : Q4Stage(args) {}
     __device__ void begin(const PrefillArgs &args, uint32_t col, int hh) {
         const PrefillGroup &g = args.group;
@@ -307,8 +307,8 @@ struct Q4GroupStage : Q4Stage {
 // then RNE to bf16.
 template <bool FIFTH>
 struct Q5Stage {
-    static constexpr int kLoads = FIFTH ? 3 : 2, kNW = 1;
-    static constexpr bool kGrouped = false;
+    static constexpr int kLoads = FIFTH ? 3 : 2, kNW = 1, kUnit = 1, kTbl = 0;
+    static constexpr bool kGrouped = false, kTall = true;
     static constexpr bool kEmit = false;
     rsrc_t p0_rsrc, p1_rsrc, m_rsrc;
     uint32_t p0_src, p1_src, m_src;
@@ -329,14 +329,14 @@ struct Q5Stage {
         m_src = ((col >> 7) * blocks * 128u + (col & 127u)) * 16u;
     }
     // 64-group g: 32-groups 2 g and 2 g + 1, block g / 4.
-    __device__ void load(uint32_t g, int set) {
+    __device__ void load(uint32_t g, int set, int) {
         p0[set] = buffer_load16_cp<2>(p0_rsrc, p0_src + g * (2u * 128u * 16u), 0);
         if constexpr (FIFTH) p1[set] = buffer_load_u32(p1_rsrc, p1_src + g * (2u * 128u * 4u), 0);
         else p1[set] = 0u;
         mr[set] = buffer_load16(m_rsrc, m_src + (g >> 2) * (128u * 16u), 0);
     }
     // Words q0 and q0 + 1: pieces q0 / 2 (elements 8 (q0 / 2) .. + 7) and 2 + q0 / 2.
-    __device__ void store(char *dst, int set, uint32_t g, bool on, int q0) {
+    __device__ void store(char *dst, int set, uint32_t g, int, bool on, int q0) {
         // Scale and minimum of 32-group j = (2 g + hh) mod 8 (GgufQuant.swift:196-203): packed byte
         // k is meta byte 4 + k; for j < 4 the low six bits of bytes 4 + j and 8 + j, else the
         // nibbles of byte 12 + (j - 4) joined with the top two bits of bytes 4 + (j - 4) and
@@ -386,8 +386,8 @@ struct Q5Stage {
 // takes differs by format, so kLoads = 0: the step's wait takes every load.
 template <int TYPE>
 struct GgufStage {
-    static constexpr int kLoads = 0, kNW = 1;
-    static constexpr bool kGrouped = false;
+    static constexpr int kLoads = 0, kNW = 1, kUnit = 1, kTbl = 0;
+    static constexpr bool kGrouped = false, kTall = true;
     static constexpr bool kEmit = false;
     rsrc_t r;
     GgufRow row;
@@ -399,9 +399,9 @@ struct GgufStage {
         const uint32_t row_bytes = (uint32_t)(args.groups * 64 / GgufGeom<TYPE>::kElems * GgufGeom<TYPE>::kBytes);
         row = gguf_row<TYPE>(col, row_bytes, args.rows32);
     }
-    __device__ void load(uint32_t g, int set) { raw[set] = gguf_fetch<TYPE>(r, row, (int)(2u * g) + hh); }
+    __device__ void load(uint32_t g, int set, int) { raw[set] = gguf_fetch<TYPE>(r, row, (int)(2u * g) + hh); }
     // The whole part at q0 = 0 (the decoders produce all 32 values at once), nothing at q0 = 2.
-    __device__ void store(char *dst, int set, uint32_t, bool on, int q0) {
+    __device__ void store(char *dst, int set, uint32_t, int, bool on, int q0) {
         if (q0 != 0) return;
         float v[32];
         gguf_decode<TYPE>(raw[set], v);
@@ -416,12 +416,47 @@ struct GgufStage {
     }
 };
 
+// The same blocks where K is whole units of 256: the thread takes half t % 2 of its column's unit, loaded
+// once for the unit's four steps (gguf_half.hpp), and step s multiplies group s of both halves, so
+// k = 32 s .. + 31 and 128 + 32 s .. + 31 of the unit. GgufStage asks for the group's own bytes every
+// step, and those of a super-block overlap (Q6_K: eight loads a thread and step, each lane in a cache line
+// of its own, the step bound by them). K5120 -> N17408, 1024 rows, ROWS32: Q6_K 250 -> 205 us, Q3_K 237 ->
+// 191, IQ3_S 289 -> 205, IQ4_XS 207 -> 190, Q8_0 216 -> 202, IQ4_NL 201 -> 190. The Q4_K and Q5_K planes, whose
+// records are coalesced as they are, gain nothing from it. At 256 rows a few of the unit's registers spill in the
+// loop; loading Q6_K's low nibbles in two parts halved that and changed nothing.
+template <int TYPE>
+struct GgufUnitStage {
+    static constexpr int kLoads = 0, kNW = 1, kUnit = 4, kTbl = Half<TYPE>::kTbl;
+    static constexpr bool kGrouped = false, kTall = GgufGeom<TYPE>::kElems == 256;
+    static constexpr bool kEmit = false;
+    Half<TYPE> half;
+    GgufSource src;
+    __device__ GgufUnitStage(const PrefillArgs &args) {
+        src = {};
+        src.w = (const uint8_t *)args.w[0];
+        src.w_bytes = args.w_bytes[0];
+        src.rows32 = args.rows32;
+        src.row_bytes = (uint32_t)(args.groups * 64 / GgufGeom<TYPE>::kElems * GgufGeom<TYPE>::kBytes);
+    }
+    __device__ void begin(const PrefillArgs &, uint32_t col, int hh) { half.start(src, col, hh); }
+    // s: g mod 4, known to the compiler.
+    __device__ void load(uint32_t g, int, int s) {
+        if (s == 0) half.load(g >> 2, true);
+    }
+    __device__ void store(char *dst, int, uint32_t, int s, bool, int q0) {
+        if (s == 0 && q0 == 0) half.take();
+        if (q0 == 0) half.group(s);
+#pragma unroll
+        for (int q = q0; q < q0 + 2; ++q) *(bf16x8 *)(dst + 16 * Half<TYPE>::piece(q)) = half.operand(q);
+    }
+};
+
 // The kernel's buffers (see the top of the file).
 // (64 FM rows.)
 constexpr int prefill_a_bytes(int fm) { return 64 * fm * 128; }
 constexpr int prefill_buf(int fm) { return prefill_a_bytes(fm) + kPABuf; }  // activations and bf16 weights of a group
-constexpr size_t prefill_lds(int fm) { return 2 * (size_t)prefill_buf(fm); }
-static_assert(8 * kPEpi <= (int)prefill_lds(2), "eight waves' epilogue staging fits the buffers");
+constexpr size_t prefill_lds(int fm, int tbl) { return 2 * (size_t)prefill_buf(fm) + tbl; }  // (tbl: after the buffers)
+static_assert(8 * kPEpi <= (int)prefill_lds(2, 0), "eight waves' epilogue staging fits the buffers");
 
 template <class W, int FM>
 __device__ __forceinline__ void prefill_body(const PrefillArgs &args) {
@@ -439,6 +474,12 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs &args) {
     const int G = (int)args.groups;
     const rsrc_t a_rsrc = make_rsrc(args.a, args.a_bytes);
     W wst(args);
+    constexpr int kUnit = W::kUnit;  // 64-element groups a job is whole multiples of
+    if constexpr (W::kTbl > 0) {
+        decltype(wst.half)::build(lds + 2 * kSBuf, tid, 512);
+        wst.half.table(lds + 2 * kSBuf);
+        lds_barrier();
+    }
     {
         // An AGPR operand makes the compiler select the AGPR form of the MFMAs: the accumulators
         // then live in AGPRs, beside a full set of 128 VGPRs.
@@ -464,7 +505,9 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs &args) {
             const int row = 64 * p + 8 * wave + (lane >> 3);
             const int piece = (lane & 7) ^ ((row >> 1) & 7);
             const int64_t m = m0 + row;
-            a_src[p] = (uint32_t)(((m < args.rows ? m : args.rows - 1) * args.lda + piece * 8) * 2);
+            // (Units of 256: pieces 4 .. 7 are the other half's.)
+            const int at = kUnit == 1 ? piece * 8 : (piece >> 2) * 128 + (piece & 3) * 8;
+            a_src[p] = (uint32_t)(((m < args.rows ? m : args.rows - 1) * args.lda + at) * 2);
         }
         // The weights of column tid / 2, k = 32 (tid % 2) .. + 31 of each group (columns past the
         // last clamped).
@@ -479,17 +522,17 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs &args) {
             return (uint32_t)__builtin_amdgcn_readfirstlane(g);
         };
         auto load_a = [&](int t, int buf) {
-            const uint32_t g = clampg(t);
+            const uint32_t g = clampg(t), at = kUnit == 1 ? g * 128u : (g >> 2) * 512u + (g & 3u) * 64u;
 #pragma unroll
             for (int p = 0; p < kAPer; ++p)
-                buffer_load_lds16(a_rsrc, lds + buf * kSBuf + 8192 * p + 1024 * wave, a_src[p] + g * 128u);
+                buffer_load_lds16(a_rsrc, lds + buf * kSBuf + 8192 * p + 1024 * wave, a_src[p] + at);
         };
-        // Group t's weights in register set t mod 2.
-        auto load_codes = [&](int t, int set) { wst.load(clampg(t), set); };
+        // Group t's weights in register set t mod 2 (s: t mod kUnit; jobs start on a unit).
+        auto load_codes = [&](int t, int set, int s) { wst.load(clampg(t), set, s); };
         // Group t's weights (half q0 / 2 of this thread's part) into buffer `buf`; zero weights
         // past the job (the step count is padded to even).
-        auto store_b = [&](int buf, int set, int t, int q0) {
-            wst.store(lds + buf * kSBuf + b_dst, set, clampg(t), t < T, q0);
+        auto store_b = [&](int buf, int set, int t, int s, int q0) {
+            wst.store(lds + buf * kSBuf + b_dst, set, clampg(t), s, t < T, q0);
         };
         // Operands of MFMA step i (k = 32 h + 8 i .. + 7 of the group, piece 4 h + i of a row).
         auto read_ops = [&](bf16x8 *af, bf16x8 *bw, int buf, int i) {
@@ -511,17 +554,19 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs &args) {
 
         // Prologue: group 0 into buffer 0, group 1's codes in flight.
         load_a(0, 0);
-        load_codes(0, 0);
-        store_b(0, 0, 0, 0);
-        store_b(0, 0, 0, 2);
+        load_codes(0, 0, 0);
+        store_b(0, 0, 0, 0, 0);
+        store_b(0, 0, 0, 0, 2);
         __builtin_amdgcn_sched_barrier(0);
-        load_codes(1, 1);
+        load_codes(1, 1, 1);
         __builtin_amdgcn_sched_barrier(0);
         wait_vmcnt<kSCodeLoads>();  // group 0's activations have landed; group 1's codes may not
         lds_barrier_staged<0>();
 
-        // Step t: buffer and code set d = t mod 2.
-        auto step = [&](int t, int d) {
+        // Step t = s modulo the unrolled steps: buffer and code set d = t mod 2.
+        constexpr int kSteps = kUnit > 2 ? kUnit : 2;
+        auto step = [&](int t, int s) {
+            const int d = s & 1;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 // Group t + 1's activations into the other buffer and group t + 2's codes, a step
@@ -529,7 +574,7 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs &args) {
                 // step); group t + 1's weights over MFMA steps 1 and 2.
                 if (i == 0) {
                     load_a(t + 1, d ^ 1);
-                    load_codes(t + 2, d);
+                    load_codes(t + 2, d, (s + 2) % kUnit);
                     __builtin_amdgcn_sched_barrier(0);
                 }
                 // No operand prefetch: the other wave on the SIMD covers the read latency.
@@ -540,7 +585,7 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs &args) {
 #pragma unroll
                     for (int f = 0; f < FM; ++f)
                         acc[f][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[f], bw[j], acc[f][j], 0, 0, 0);
-                if (i == 1 || i == 2) store_b(d ^ 1, d ^ 1, t + 1, 2 * (i - 1));
+                if (i == 1 || i == 2) store_b(d ^ 1, d ^ 1, t + 1, (s + 1) % kUnit, 2 * (i - 1));
             }
             // Group t + 1's activations have landed (only group t + 2's code loads, issued after
             // them, may be outstanding), and every wave is done with buffer t mod 2.
@@ -548,10 +593,14 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs &args) {
             wait_vmcnt<kSCodeLoads>();
             lds_barrier_staged<0>();
         };
-        const int Tp = (T + 1) / 2 * 2;
-        for (int t0 = 0; t0 < Tp; t0 += 2) {
+        const int Tp = (T + kSteps - 1) / kSteps * kSteps;
+        for (int t0 = 0; t0 < Tp; t0 += kSteps) {
             step(t0, 0);
             step(t0 + 1, 1);
+            if constexpr (kSteps == 4) {
+                step(t0 + 2, 2);
+                step(t0 + 3, 3);
+            }
         }
         const int64_t ncol = n0 + ((64 * wn) & (kTileCols - 1));  // the wave's first output column
         if (NW == 2 && slot < 0)
@@ -577,11 +626,14 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs &args) {
             job_slot = -1;
             dp_tile += P;
         } else if (u < u_end) {
-            tile = args.dp_tiles + (int)(u / G);
-            ga = (int)(u % G);
-            gb = (int)((int64_t)ga + (u_end - u) < G ? ga + (u_end - u) : G);
+            // (args.sk_units counts units.)
+            const int U = G / kUnit, ua = (int)(u % U);
+            const int ub = (int)((int64_t)ua + (u_end - u) < U ? ua + (u_end - u) : U);
+            tile = args.dp_tiles + (int)(u / U);
+            ga = ua * kUnit;
+            gb = ub * kUnit;
             job_slot = (ga == 0 && gb == G) ? -1 : slot;
-            u += gb - ga;
+            u += ub - ua;
             slot = 1;
         } else {
             break;
@@ -755,11 +807,14 @@ PrefillPlan plan_prefill(int64_t rows, int64_t columns, int64_t groups, size_t w
     return best;
 }
 
+size_t prefill_plan_bytes(const PrefillPlan &plan) {
+    return plan.sk_units > 0 ? prefill_sk_bytes(plan.sk_grid, plan.fm) : 0;
+}
+
 size_t prefill_workspace_bytes(int64_t rows, int64_t columns, int64_t groups) {
     size_t need = 0;
-    for (const double decode : {kPrefillDecodeQ4, kPrefillDecodePlanes, kPrefillDecodeNative}) {
-        const PrefillPlan p = plan_prefill(rows, columns, groups, (size_t)-1, decode);
-        const size_t bytes = p.sk_units > 0 ? prefill_sk_bytes(p.sk_grid, p.fm) : 0;
+    for (const double decode : {kPrefillDecodeQ4, kPrefillDecodePlanes, kPrefillDecodeNative, kPrefillDecodeUnits}) {
+        const size_t bytes = prefill_plan_bytes(plan_prefill(rows, columns, groups, (size_t)-1, decode));
         need = need > bytes ? need : bytes;
     }
     return need;
@@ -781,28 +836,28 @@ static hipError_t launch_prefill(const PrefillPlan &plan, PrefillArgs &args, int
     args.mblocks = plan.mblocks;
     args.partial = plan.sk_units > 0 ? (float *)((char *)workspace + kPCounterBytes) : nullptr;
     args.dp_tiles = plan.dp_tiles;
-    args.sk_units = plan.sk_units;
+    args.sk_units = plan.sk_units / W::kUnit;
     args.a_bytes = (uint32_t)(((rows - 1) * lda + inner) * 2);
     args.sk_grid = plan.sk_grid;
     void (*high)(PrefillArgs);
-    if constexpr (W::kGrouped) high = prefill_tile_kernel<W, 4>;
-    else high = prefill_kernel<W>;
+    if constexpr (W::kTall) high = prefill_kernel<W>;
+    else high = prefill_tile_kernel<W, 4>;
     static const bool once = [&] {
         (void)hipFuncSetAttribute((const void *)prefill_tile_kernel<W, 2>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  (int)prefill_lds(2));
+                                  (int)prefill_lds(2, W::kTbl));
         (void)hipFuncSetAttribute((const void *)prefill_tile_kernel<W, 3>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  (int)prefill_lds(3));
-        (void)hipFuncSetAttribute((const void *)high, hipFuncAttributeMaxDynamicSharedMemorySize, (int)prefill_lds(4));
+                                  (int)prefill_lds(3, W::kTbl));
+        (void)hipFuncSetAttribute((const void *)high, hipFuncAttributeMaxDynamicSharedMemorySize, (int)prefill_lds(4, W::kTbl));
         return true;
     }();
     (void)once;
     const auto kernel = plan.fm == 2 ? prefill_tile_kernel<W, 2> : plan.fm == 3 ? prefill_tile_kernel<W, 3> : high;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)plan.grid), dim3(512), prefill_lds(plan.fm), stream, args);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)plan.grid), dim3(512), prefill_lds(plan.fm, W::kTbl), stream, args);
     hipError_t err = hipGetLastError();
     if (err != hipSuccess || plan.sk_units == 0) return err;
     const int remainder = plan.tiles - plan.dp_tiles;
     hipLaunchKernelGGL(prefill_finish, dim3((unsigned)remainder, 64 * plan.fm * kPB / 1024 / W::kNW), dim3(256), 0,
-                       stream, (const float *)args.partial, plan.dp_tiles, plan.sk_units, plan.sk_grid, args.groups,
+                       stream, (const float *)args.partial, plan.dp_tiles, args.sk_units, plan.sk_grid, args.groups / W::kUnit,
                        plan.mblocks, 64 * plan.fm, rows, n, out, ldc, out_dtype, residual, W::kNW, args.emit, args.group);
     return hipGetLastError();
 }
@@ -904,15 +959,15 @@ hipError_t launch_gguf_prefill(const PrefillPlan &plan, int type, const uint8_t 
     args.rows32 = gguf_layout(type);
     args.w[0] = native;
     args.w_bytes[0] = (uint32_t)((args.rows32 ? (rows_w + 31) / 32 * 32 : rows_w) * (inner / elems) * bytes);
-#define SPLOSH_GGUF_PREFILL(T) \
-    launch_prefill<GgufStage<T>>(plan, args, rows_w, inner, a, lda, out, ldc, out_dtype, residual, rows, workspace, stream)
+#define SPLOSH_GGUF_PREFILL(STAGE) \
+    launch_prefill<STAGE>(plan, args, rows_w, inner, a, lda, out, ldc, out_dtype, residual, rows, workspace, stream)
     switch (type) {
-        case 8: return SPLOSH_GGUF_PREFILL(8);
-        case 11: return SPLOSH_GGUF_PREFILL(11);
-        case 14: return SPLOSH_GGUF_PREFILL(14);
-        case 20: return SPLOSH_GGUF_PREFILL(20);
-        case 21: return SPLOSH_GGUF_PREFILL(21);
-        default: return SPLOSH_GGUF_PREFILL(23);
+        case 8: return inner % 256 == 0 ? SPLOSH_GGUF_PREFILL(GgufUnitStage<8>) : SPLOSH_GGUF_PREFILL(GgufStage<8>);
+        case 20: return inner % 256 == 0 ? SPLOSH_GGUF_PREFILL(GgufUnitStage<20>) : SPLOSH_GGUF_PREFILL(GgufStage<20>);
+        case 11: return SPLOSH_GGUF_PREFILL(GgufUnitStage<11>);
+        case 14: return SPLOSH_GGUF_PREFILL(GgufUnitStage<14>);
+        case 21: return SPLOSH_GGUF_PREFILL(GgufUnitStage<21>);
+        default: return SPLOSH_GGUF_PREFILL(GgufUnitStage<23>);
     }
 #undef SPLOSH_GGUF_PREFILL
 }

@@ -18,7 +18,8 @@ def test_tile_kernels_wait_for_their_loads(tmp_path):
                     str(wc.ROOT / "splosh_amd" / "csrc" / "prefill.hip"), "-o", str(out)], check=True,
                    capture_output=True)
     kernels = list(wc._kernels(out.read_text(), r"_ZN6splosh19prefill_tile_kernel\S*"))
-    assert len(kernels) == 2 * 10 + 3  # two lower tiles of every stage, three of the grouped one
+    # Two lower tiles of ten stages, three of the grouped one and of Q8_0 and IQ4_NL in whole units.
+    assert len(kernels) == 2 * 10 + 3 + 2 * 3
     for name, code in kernels:
         assert any(wc._is_lds(ins) for ins in code), name
         fm = int(re.search(r"Li(\d)EEEvNS_11PrefillArgs", name).group(1))
