@@ -86,6 +86,13 @@ bool q4_stream_eligible(const splosh_q4_weight &w, const uint16_t *a, int64_t ld
     return true;
 }
 
+// 80..128 rows of a weight this large (elements): one call of the prefill kernel (128-row tiles) instead of
+// two of at most 64 rows, given its scratch. Two calls / one (us): K5120 -> N17408 at 65 rows 42.9 / 46.1, 80
+// 44.4 / 43.6, 96 49.6 / 44.1, 128 54.4 / 45.2; its gate+up 67.5 / 69.6, 69.3 / 66.5, 75.4 / 67.8, 85.9 / 74.1;
+// K17408 -> N5120 41.0 / 44.4, 49.6 / 43.1, 46.8 / 43.6, 52.1 / 44.1. Not the smaller ones: K5120 -> N12288 at
+// 96 rows 32.9 / 34.8, N5120 25.7 / 27.7.
+constexpr int64_t kPrefillLargeWeight = 80 << 20, kPrefillLargeRows = 80;
+
 int q4_gemm_impl(const splosh_q4_weight *w, const splosh_q4_weight *up, const uint16_t *a, int64_t lda, void *out,
                  int64_t ldc, int out_dtype, const void *residual, int64_t rows, int kernel, void *workspace,
                  size_t workspace_bytes, hipStream_t stream, const splosh::EmitOperand *emit = nullptr,
@@ -107,11 +114,18 @@ int q4_gemm_impl(const splosh_q4_weight *w, const splosh_q4_weight *up, const ui
         splosh::rows_fit(rows, w->rows, w->inner, lda))
         return hip_status(splosh::launch_q4_rows(*w, a, lda, out, ldc, out_dtype, residual, rows, stream),
                           "q4 rows launch");
-    // 65..128 rows under AUTO: rows 0..63 and the rest as two calls of the M <= 64 kernels, one after
-    // the other on the stream (the workspace's counters are zero again between them). Measured at
-    // K5120 -> 2 x N17408 (gate+up) and K17408 -> N5120, against the one call on the tile or
-    // prefill kernel: gate+up M=65 91 -> 60 us, M=96 94 -> 72, M=128 97 -> 80; down M=65 54 -> 38,
-    // M=96 55 -> 47, M=128 58 -> 51; at 192 rows three calls lose (120 against 104 us).
+    if (kernel == SPLOSH_KERNEL_AUTO && !emit && wide16 && w->order == SPLOSH_Q4_TILED128 &&
+        rows >= kPrefillLargeRows && rows <= 128 && w->rows * w->inner >= kPrefillLargeWeight && aligned(out, 16) &&
+        (!residual || aligned(residual, 16)) && splosh::prefill_fits(rows, w->rows, w->inner, lda, ldc)) {
+        const size_t need = splosh::prefill_plan_bytes(
+            splosh::plan_prefill(rows, (up ? 2 : 1) * w->rows, w->inner / kGroupSize, (size_t)-1));
+        if (need == 0 || (workspace && workspace_bytes >= need)) kernel = SPLOSH_KERNEL_PREFILL;
+    }
+    // Else 65..128 rows under AUTO: rows 0..63 and the rest as two calls of the M <= 64 kernels, one after
+    // the other on the stream (the workspace's counters are zero again between them). Two calls / one
+    // of the prefill kernel at 65, 96 and 128 rows (us): K5120 -> N5120 22.0 / 25.8, 25.7 / 27.7,
+    // 29.2 / 30.2; N7168 22.9 / 27.3, 27.3 / 30.2, 31.9 / 32.6; at 192 rows three calls lose (gate+up
+    // 120 against 96).
     if (kernel == SPLOSH_KERNEL_AUTO && !emit && rows > 64 && rows <= 128 && wide16 &&
         splosh::mma_fits(64, w->rows, w->inner, w->row_stride_words, lda)) {
         const char *res = (const char *)residual;
