@@ -70,7 +70,8 @@ typedef enum splosh_kernel {
                                    without a barrier in its loop; else up to 64: DEQUANT (a single weight of at least two
                                    64-column bands a CU as the pair of its column halves); 65..128:
                                    rows 0..63 and the rest as two calls of the above (without the
-                                   emit); more: PREFILL for tiled weights with lda % 8 == 0 and
+                                   emit; PREFILL from 80 rows of tiled weights of 80 Mi elements,
+                                   given its scratch); more: PREFILL for tiled weights with lda % 8 == 0 and
                                    ldc % 4 == 0, else TILE; SCALAR for operands no other kernel
                                    takes. A row-major weight of one or two rows, or of few outputs
                                    (rows.hip), takes a latency-shaped kernel of its own first */
@@ -85,9 +86,9 @@ typedef enum splosh_kernel {
     SPLOSH_KERNEL_SCALAR = 4,   /* one thread per output (gemm_q4.metal semantics) */
     SPLOSH_KERNEL_PREFILL = 5   /* TILED128 q4 weights (mlp_in: 128 columns of each a tile,
                                    silu(g) * u in the epilogue) or Q5_K / Q4_K planes:
-                                   256 x 256 output tiles, two waves per SIMD, every weight
+                                   128 to 256 x 256 output tiles, two waves per SIMD, every weight
                                    dequantized once a tile into LDS; uses the workspace to split
-                                   the last round of tiles over all CUs */
+                                   the remaining tiles over K */
 } splosh_kernel;
 
 /* Q4BufferLayout (Quant/Q4BufferLayout.swift:29-79). */
@@ -246,7 +247,7 @@ int splosh_untile128(const void *src, void *dst, int64_t rows, int64_t groups, i
 /* Engine.gemm on a GGUF weight (Runtime/Engine.swift:1671-1697, kernels
  * Shaders/engine_gguf.metal:82-221 instantiated _q5k at :332-349). AUTO: one row takes the
  * every-CU decode kernel; 2..64 rows the dequant-to-bf16 MFMA kernel (DEQUANT; lda % 8 == 0 and
- * 16-byte aligned activations), 65..128 rows two calls of at most 64; more rows the 256 x 256
+ * 16-byte aligned activations), 65..128 rows two calls of at most 64; more rows the 256-column
  * prefill kernel (PREFILL; also ldc % 4 == 0
  * and 16-byte aligned outputs), else the LDS-tiled kernel (TILE), else the streaming kernel
  * (STREAM). DEQUANT and PREFILL use a workspace of splosh_workspace_bytes(rows, w->rows, w->inner)
@@ -316,13 +317,14 @@ int splosh_q4k_dequant(const splosh_q5k_weight *w, float *out, hipStream_t strea
  * order scatters over 32 rows (at K17408 -> N5120, M=64: Q8_0 44 -> 33 us, IQ4_XS 39 -> 31).
  *
  * splosh_gguf_gemm: out[m][n] = sum_k a[m][k] w[n][k] (+ residual). Up to a few activation rows
- * (IQ4_NL 3, Q3_K 6, the others 4) a streaming kernel reads the weight once. Up to 64 rows
- * (inner % 256 == 0) the stream-K MFMA kernel of splosh_q4_gemm decodes each weight group once,
- * and 65..128 rows run as two such calls but for Q3_K (where it does not fit, the streaming kernel
- * serves up to eight rows). Above that an LDS-tiled
- * MFMA kernel (inner % 64 == 0) decodes each weight group once per 64 or 128 activation rows. From 256
- * rows (rows % 128 == 0, ldc % 4 == 0, 16-byte aligned outputs) the 256 x 256 prefill kernel
- * decodes each group once per 256 rows. The MFMA kernels split K over workgroups when their work
+ * a streaming kernel reads the weight once, or, where it is the faster up to 16 or 32 rows, a
+ * barrier-free MFMA kernel (inner % 256 == 0). Up to 64 rows (inner % 256 == 0) the stream-K MFMA
+ * kernel of splosh_q4_gemm decodes each weight group once, and 65..128 rows run as two such calls
+ * (where it does not fit, the streaming kernel serves up to eight rows). The prefill kernel (rows % 128
+ * == 0, ldc % 4 == 0, 16-byte aligned outputs) decodes each group once per 128 to 256 activation rows: from
+ * 256 rows, with inner % 256 == 0 and its scratch from 129, for Q3_K and weights of 40 Mi elements from
+ * 65. Else, above 64 rows, an LDS-tiled MFMA kernel (inner % 64 == 0) decodes each weight group once per 64 or
+ * 128 rows. The MFMA kernels split K over workgroups when their work
  * is uneven or their tiles few and a workspace of splosh_workspace_bytes(m, rows, inner) is given
  * (zero-filled before first use; the kernels leave their counters zeroed, so one workspace serves
  * every later call; null: no split).

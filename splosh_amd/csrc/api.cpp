@@ -726,7 +726,7 @@ static int gguf_gemm(const splosh_q5k_weight *w_in, bool fifth, const uint16_t *
     if (kernel == SPLOSH_KERNEL_AUTO) {
         if (!eligible) choice = SPLOSH_KERNEL_SCALAR;
         else if (mma_ok) choice = SPLOSH_KERNEL_DEQUANT;
-        // Above 64 rows the 256 x 256 prefill kernel (K17408 -> N5120: 75 us at 128 rows against the
+        // Above 64 rows the prefill kernel (K17408 -> N5120: 75 us at 128 rows against the
         // tile kernel's 86, 381 against 627 at 2048).
         else if (prefill_ok) choice = SPLOSH_KERNEL_PREFILL;
         else if (tile_ok) choice = SPLOSH_KERNEL_TILE;
