@@ -40,15 +40,16 @@ struct HalfNative {
     __device__ static void build(char *, int, int) {}
     __device__ void table(const char *) {}
 };
-// Codes 0 .. 255 of group word pair 2 i with scale s and offset o: s code + o in one rounding.
-__device__ __forceinline__ bf16x8 sg_bytes(const uint32_t (&wd)[8], int i, float s, float o) {
+// Codes 0 .. 255 of group word pair 2 i: s (code - zero), the difference exact, in one rounding (and with
+// the decoder's infinities and NaN, which an fma with an offset of -zero s would not keep).
+__device__ __forceinline__ bf16x8 sg_bytes(const uint32_t (&wd)[8], int i, float s, float zero) {
     u32x4 d;
 #pragma unroll
     for (int q = 0; q < 2; ++q)
 #pragma unroll
         for (int e = 0; e < 2; ++e)
-            d[2 * q + e] = f32x2_to_bf16x2(__builtin_fmaf(cvt_byte(wd[2 * i + q], 2 * e), s, o),
-                                           __builtin_fmaf(cvt_byte(wd[2 * i + q], 2 * e + 1), s, o));
+            d[2 * q + e] = f32x2_to_bf16x2(s * (cvt_byte(wd[2 * i + q], 2 * e) - zero),
+                                           s * (cvt_byte(wd[2 * i + q], 2 * e + 1) - zero));
     return as_bf16x8(d);
 }
 // Dword k of bytes that start 2 bytes into a.
@@ -73,8 +74,7 @@ struct Half<8> : HalfNative {  // Q8_0: four blocks of fp16 d and 32 int8 codes 
 #pragma unroll
         for (int q = 0; q < 8; ++q) wd[q] = (j & 1 ? x[(34 * j + 2) / 4 + q] : mid(x, 34 * j / 4 + q)) ^ 0x80808080u;
     }
-    // d c as d (c + 128) - 128 d: the product's one rounding (128 d is exact).
-    __device__ bf16x8 operand(int i) const { return sg_bytes(wd, i, s0, -128.0f * s0); }
+    __device__ bf16x8 operand(int i) const { return sg_bytes(wd, i, s0, 128.0f); }
 };
 
 template <>
@@ -111,10 +111,9 @@ struct Half<14> : HalfNative {  // Q6_K: ql[128], qh[64], scales[16], d (:218-23
         for (int q = 0; q < 8; ++q)
             wd[q] = ((xl[8 * (j & 1) + q] >> (4 * (j >> 1))) & 0x0F0F0F0Fu) | (((xh[q] >> (2 * j)) & 0x03030303u) << 4);
     }
-    // ds (c - 32) as one fma (-32 ds is exact).
     __device__ bf16x8 operand(int i) const {
         const float s = i < 2 ? s0 : s1;
-        return sg_bytes(wd, i, s, -32.0f * s);
+        return sg_bytes(wd, i, s, 32.0f);
     }
 };
 
@@ -154,7 +153,7 @@ struct Half<11> : HalfNative {  // Q3_K: hmask[32], qs[64], scales[12], d (:238-
     }
     __device__ bf16x8 operand(int i) const {
         const float s = i < 2 ? s0 : s1;
-        return sg_bytes(wd, i, s, -4.0f * s);
+        return sg_bytes(wd, i, s, 4.0f);
     }
 };
 
