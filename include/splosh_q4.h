@@ -317,12 +317,14 @@ int splosh_q4k_dequant(const splosh_q5k_weight *w, float *out, hipStream_t strea
  * order scatters over 32 rows (at K17408 -> N5120, M=64: Q8_0 44 -> 33 us, IQ4_XS 39 -> 31).
  *
  * splosh_gguf_gemm: out[m][n] = sum_k a[m][k] w[n][k] (+ residual). Up to a few activation rows
- * a streaming kernel reads the weight once, or, where it is the faster up to 16 or 32 rows, a
- * barrier-free MFMA kernel (inner % 256 == 0). Up to 64 rows (inner % 256 == 0) the stream-K MFMA
+ * (IQ4_NL 3, Q3_K 6, the others 4) a streaming kernel reads the weight once and rounds no weight;
+ * above, the kernels round the decoded weights to bf16. Up to 16 or 32 rows a barrier-free MFMA
+ * kernel (inner % 256 == 0) where it is the fastest; up to 64 rows (inner % 256 == 0) the stream-K MFMA
  * kernel of splosh_q4_gemm decodes each weight group once, and 65..128 rows run as two such calls
  * (where it does not fit, the streaming kernel serves up to eight rows). The prefill kernel (rows % 128
  * == 0, ldc % 4 == 0, 16-byte aligned outputs) decodes each group once per 128 to 256 activation rows: from
- * 256 rows, with inner % 256 == 0 and its scratch from 129, for Q3_K and weights of 40 Mi elements from
+ * 256 rows, with inner % 256 == 0 and its scratch from 129, for weights of 40 Mi elements from 69 (IQ4_NL
+ * 68), for Q3_K from
  * 65. Else, above 64 rows, an LDS-tiled MFMA kernel (inner % 64 == 0) decodes each weight group once per 64 or
  * 128 rows. The MFMA kernels split K over workgroups when their work
  * is uneven or their tiles few and a workspace of splosh_workspace_bytes(m, rows, inner) is given

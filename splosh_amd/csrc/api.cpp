@@ -850,7 +850,7 @@ constexpr int64_t kGgufPrefillRows = 256;  // measured: the tile kernel is as fa
 // Rows from which weights of whole 256-element units take it instead, given the scratch of its plan: above
 // the two calls of the M <= 64 kernel (K17408 -> N5120 at 160 rows, tiled kernel and this: Q6_K 130 -> 61 us,
 // IQ3_S 160 -> 60, IQ4_XS 114 -> 56, Q8_0 125 -> 62; K1536 -> N4096 37..41 -> 23..26), and from 65 rows for the
-// weights where it wins over those: the large ones (K5120 -> N17408 at 65 and 128 rows: Q6_K 69 / 96 -> 59 / 66,
+// weights where it wins over those: the large ones (but the exact rows past 64; K5120 -> N17408 at 65 and 128 rows: Q6_K 69 / 96 -> 59 / 66,
 // IQ4_XS 57 / 75 -> 51 / 57, Q8_0 65 / 80 -> 58 / 65; K11008 -> N4096 41 / 57 -> 35 / 38; but K1536 -> N11008
 // 20 / 22 -> 24 / 27 and K5120 -> N5120 26.9 / 36 -> 27.9 / 29), and Q3_K (the tiled kernel before: 84 / 87 ->
 // 49 / 55, K1536 -> N4096 24 / 24 -> 18 / 22).
@@ -874,8 +874,10 @@ static int gguf_native_gemm(int gguf_type, const uint8_t *native, int64_t rows, 
     // 47, IQ3_S 42, IQ4_NL 27, IQ4_XS 30); the streaming kernel at four rows Q8_0 31, Q6_K 35, Q3_K
     // 32, IQ3_S 31, IQ4_NL 29, IQ4_XS 29, at five Q6_K 45, Q3_K 43, IQ3_S 43, at six Q3_K 47, at
     // three IQ4_NL 26. Where the MFMA kernel does not fit (K % 256 != 0), the streaming kernel
-    // serves up to eight rows and the LDS-tiled kernel above. Up to 32 rows the barrier-free kernel of
-    // skinny_gguf.hip comes first where it is the faster. (A development override of the
+    // serves up to eight rows and the LDS-tiled kernel above. From the streaming limit to 32 rows the
+    // barrier-free kernel of skinny_gguf.hip comes first where it is the faster; up to the limit the weights
+    // enter the sums exactly, so it does not, though it would be the faster at large weights (K17408 -> N5120,
+    // two to four rows: Q8_0 27 to 28 us against 33 to 36). (A development override of the
     // prefill threshold, read once.)
     static const int64_t prefill_rows = [] {
         const char *e = getenv("SPLOSH_GGUF_PREFILL_ROWS");
@@ -884,9 +886,12 @@ static int gguf_native_gemm(int gguf_type, const uint8_t *native, int64_t rows, 
     const bool units = inner % 256 == 0;
     const double decode = units ? splosh::kPrefillDecodeUnits : splosh::kPrefillDecodeNative;
     const int base_type = gguf_type & 0xFF;
-    const int64_t from = !units ? prefill_rows
-                         : base_type == 11 || rows * inner >= kGgufPrefillLargeWeight ? 65
-                                                                                      : kGgufPrefillUnitRows;
+    const int64_t stream_max = base_type == 11 ? 6 : base_type == 20 ? 3 : 4;
+    // (The rows past 64 of a call of two are exact up to stream_max of them: the prefill kernel from the next.)
+    const int64_t from = !units                                    ? prefill_rows
+                         : base_type == 11                         ? 65
+                         : rows * inner >= kGgufPrefillLargeWeight ? 65 + stream_max
+                                                                   : kGgufPrefillUnitRows;
     bool prefill = m >= (from < prefill_rows ? from : prefill_rows) && aligned(out, 16) &&
                    (!residual || aligned(residual, 16)) &&
                    splosh::gguf_prefill_fits(gguf_type, m, rows, inner, lda, ldc);
@@ -896,7 +901,6 @@ static int gguf_native_gemm(int gguf_type, const uint8_t *native, int64_t rows, 
                                           m, rows, inner / kGroupSize, (size_t)-1, decode));
         prefill = need == 0 || (workspace && workspace_bytes >= need);
     }
-    const int64_t stream_max = base_type == 11 ? 6 : base_type == 20 ? 3 : 4;
     // 65..128 rows: two calls of at most 64 rows, as for q4. K17408 -> N5120, against the tiled
     // kernel: M=96 Q8_0 80 -> 77 us (ROWS32 79 -> 66), Q6_K 100 -> 90, IQ3_S 105 -> 89, IQ4_NL 81 ->
     // 63, IQ4_XS 81 -> 70; Q3_K, whose MFMA path is the slowest, 83 -> 96, keeps the tiled kernel where the
@@ -914,8 +918,8 @@ static int gguf_native_gemm(int gguf_type, const uint8_t *native, int64_t rows, 
     int elems = 0, bytes = 0;
     splosh::gguf_native_block(base_type, &elems, &bytes);
     const int64_t stored = (gguf_type & SPLOSH_GGUF_ROWS32) ? (rows + 31) / 32 * 32 : rows;
-    // (A head-ordered call the streaming kernel takes stays there: it needs no workspace.)
-    const bool skinny = !(ho.on() && m <= stream_max) &&
+    // (Up to stream_max rows the weights enter the sums exactly, and a head-ordered call needs no workspace.)
+    const bool skinny = m > stream_max &&
                         splosh::gguf_skinny_fits(gguf_type, m, rows, inner, lda, stored * (inner / elems * bytes));
     const bool mma = !prefill && !skinny && m > stream_max && splosh::gguf_mma_fits(gguf_type, m, rows, inner, lda);
     const bool tile = !prefill && !skinny && !mma && m > 8 && splosh::gguf_tile_fits(m, rows, inner, lda);

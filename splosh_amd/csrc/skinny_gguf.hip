@@ -203,18 +203,18 @@ static bool sg_shape(int64_t rows, int64_t columns, int64_t inner, int64_t lda) 
            (rows * lda + inner) * 2 < ((int64_t)1 << 30);
 }
 
-// And the calls it is the fastest for (us, K17408 -> N5120, file order, this kernel against the kernel
+// And the calls it is the fastest for (native blocks: of those past the streaming kernels' rows, whose
+// weights are not rounded; us, K17408 -> N5120, file order, this kernel against the kernel
 // before it): 5 to 16 rows of every type (8 rows: Q8_0 30.3 / 33.1, Q6_K 27.9 / 43.0, Q3_K 21.6 /
 // 46.1, IQ3_S 26.2 / 42.4, IQ4_NL 23.3 / 27.2, IQ4_XS 23.0 / 30.0, Q4_K 18.7 / 21.8, Q5_K 21.4 /
-// 23.8); two to four rows, and one of Q3_K (20.5 / 22.0), from about the size of K5120 -> N3328 (8.9
-// against 8.3 on the streaming kernel at N1024, 11.4 against 14.2 at N5120); 17 to 32 rows, where
+// 23.8); two to four rows of the planes (K5120 -> N3328: Q4_K 8.4 / 11.6, Q5_K 9.9 / 12.3; N2560, below
+// the line, on mma.hip 11.0 and 11.9) and four of IQ4_NL, from 2048 blocks x units; 17 to 32 rows, where
 // the activations' traffic grows, of the types whose loads weigh most in mma.hip (32 rows: Q6_K 39.2 /
 // 43.2, Q3_K 31.8 / 46.3, IQ3_S 35.4 / 42.8, IQ4_XS in the file's order 32.3 / 34.1; not Q8_0 41.0 / 38.6).
 bool gguf_skinny_fits(int type, int64_t rows, int64_t columns, int64_t inner, int64_t lda, int64_t weight_bytes) {
     if (!sg_shape(rows, columns, inner, lda) || weight_bytes >= (int64_t)kSgOut - 65536) return false;
     const bool rows32 = gguf_layout(type);
-    if (rows <= 4)
-        return (rows > 1 || type == 11) && (columns + kSgCols - 1) / kSgCols * (inner / 256) >= 2048;
+    if (rows <= 4) return rows > 1 && (columns + kSgCols - 1) / kSgCols * (inner / 256) >= 2048;
     return rows <= 16 || type == 14 || type == 11 || type == 21 || (type == 23 && !rows32);
 }
 
