@@ -26,6 +26,7 @@
 //    (balance_merge, common.hpp).
 #include "common.hpp"
 #include "launch.hpp"
+#include "mix.hpp"
 
 namespace splosh {
 
@@ -85,8 +86,10 @@ struct SkinnyShape {
 enum SkinnyMode { kSkinnyOne, kSkinnyGroup, kSkinnySplit, kSkinnyMlp };
 constexpr int skinny_nw(SkinnyMode mode) { return mode >= kSkinnySplit ? 2 : 1; }
 
+// (Registers: two workgroups of eight waves a CU up to 16 rows, which the K slices of a long K count on; K17408
+// -> N5120 at 12 to 16 rows 22.9 us with one, 18.4 with two.)
 template <SkinnyMode MODE, int RM, int KW, int D>
-__global__ void __launch_bounds__(KW * 64, skinny_nw(MODE) == 2 ? 3 : 4)
+__global__ void __launch_bounds__(KW * 64, skinny_nw(MODE) == 2 && RM == 32 ? 3 : 4)
 q4_skinny_kernel(SkinnyArgs args) {
     constexpr int NW = skinny_nw(MODE);
     using S = SkinnyShape<RM, KW, D>;
@@ -199,6 +202,8 @@ q4_skinny_kernel(SkinnyArgs args) {
                                      sk_and_or(q >> 8, kMask, magic), sk_and_or(q >> 12, kMask, magic)};
                     prod[w] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x[i], as_bf16x8(b), prod[w], 0, 0, 0);
                 }
+                // (Keeps the second half's operands from being built early: 28 bytes a lane spilled at 8 rows.)
+                if (NW == 2 && i == 1) __builtin_amdgcn_sched_barrier(0);
             }
 #pragma unroll
             for (int w = 0; w < NW; ++w) {
@@ -214,12 +219,46 @@ q4_skinny_kernel(SkinnyArgs args) {
         }
     }
     wait_vmcnt<0>();
+    float probe = 0.0f;  // NaN if a sum of this lane is infinite or NaN
+#pragma unroll
+    for (int w = 0; w < NW; ++w)
+#pragma unroll
+        for (int e = 0; e < E; ++e) probe = __builtin_fmaf(acc[w][e], 0.0f, probe);
     __syncthreads();  // every load into LDS has landed: the sums take its place
     float *red = (float *)lds;
 #pragma unroll
     for (int w = 0; w < NW; ++w)
 #pragma unroll
         for (int e = 0; e < E; ++e) red[((wave * NW + w) * E + e) * 64 + lane] = acc[w][e];
+    // An infinite activation or scale leaves inf - inf in s P + (b - 128 s) S, and one above 2^120 can overflow
+    // it where x w does not: a wave with such a sum goes over its groups again with the dequantized weights (as
+    // mma.hip) and takes the new sums in the place of those. No finite sum changes. (Here, with the sums in LDS,
+    // it costs a call without such values less than 1%; before they leave the registers 1 to 5%.)
+    if (__builtin_expect(__ballot(probe != probe) != 0, 0)) {
+        const uint32_t row = r < args.rows ? (uint32_t)(r * args.lda * 2) : kRowOut;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+            f32x16 again = zero;
+#pragma unroll 1
+            for (int g = ga + wave; g < gb; g += KW) {
+                const uint32_t rec = rec0 + (uint32_t)g * 128u;
+                const u32x4 q = buffer_load16(q_rsrc[w], rec * 32u + 16u * h, 0);
+                const float s = bf16_bits_to_f32(buffer_load_u16(s_rsrc[w], rec * 2u, 0));
+                const float b = bf16_bits_to_f32(buffer_load_u16(b_rsrc[w], rec * 2u, 0));
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const u32x4 x = buffer_load16(a_rsrc, row + (uint32_t)g * 128u + 16u * (4 * h + i), 0);
+                    again = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(x), dequant_word_fp8(q[i], s, b), again, 0, 0, 0);
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                float *sum = red + ((wave * NW + w) * E + e) * 64 + lane;
+                const float none = *sum * 0.0f;
+                if (none != none) *sum = again[e];
+            }
+        }
+    }
     __syncthreads();
     // Thread t takes outputs t, t + kThreads, ... of the block's E x 64 in the MFMA's layout.
     constexpr int V = S::kVals;
