@@ -117,3 +117,9 @@ def test_pair(rt, rows, n, k):
         with np.errstate(invalid="ignore", over="ignore"):
             g, u = reference(bits, gate.dense), reference(bits, up.dense)
             check(got, g * (1 / (1 + np.exp(-g))) * u, f"pair {rows} {n} {k} {value} {place}")
+
+
+# Row-major weights: the dot kernel with 1 x 1, 1 x 2 and 2 x 4 outputs a workgroup, K over one round.
+@pytest.mark.parametrize("rows,n,k", [(3, 48, 1088), (2, 1024, 5120), (33, 48, 192), (5, 481, 320), (64, 96, 8256)])
+def test_row_major_few_outputs(rt, rows, n, k):
+    check_weight(rt, n, k, rows, tiled=False)
