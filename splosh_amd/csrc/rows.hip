@@ -247,14 +247,14 @@ q4_rows_mma_kernel(RowsArgs args) {
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[e] = 0.0f;
     const int G = args.groups;
-    // Group g of the wave in buffer `buf`, the next one on its way into the other. A group past the
-    // last (at most 15 past; wave-uniform) is clamped into the weight and multiplied by zero.
+    // Group g of the wave in buffer `buf`, the next one (past the last: clamped, and not multiplied) on its way
+    // into the other.
     auto clamp = [&](int g) { return g < G ? g : G - 1; };
     auto step = [&](int g, int buf) {
         load(buf ^ 1, clamp(g + kRowsMmaWaves));
         wait_vmcnt<kLoads>();  // this group has landed; the next may be in flight
         asm volatile("" ::: "memory");
-        const float sc = g < G ? bf16_bits_to_f32(s[buf]) : 0.0f, bi = g < G ? bf16_bits_to_f32(b[buf]) : 0.0f;
+        const float sc = bf16_bits_to_f32(s[buf]), bi = bf16_bits_to_f32(b[buf]);
         const char *a = mine + buf * kRowsTile + r * 128;
 #pragma unroll
         for (int i = 0; i < 4; ++i)
@@ -268,6 +268,7 @@ q4_rows_mma_kernel(RowsArgs args) {
         load(0, wave);
         for (int g = wave; g < G; g += 2 * kRowsMmaWaves) {
             step(g, 0);
+            if (g + kRowsMmaWaves >= G) break;
             step(g + kRowsMmaWaves, 1);
         }
     }
@@ -298,7 +299,7 @@ q4_rows_mma_kernel(RowsArgs args) {
 // 26); up to kRowsDotOutputs outputs of at most kRowsDotColumns columns on the same kernel
 // (N=48: 16 rows 10.0 -> 3.0 us, 64 rows 12 -> 4.7, 333 rows 19 -> 12; N=512, 16 rows 12.2 -> 7.5;
 // at 16384 outputs and 64 rows or fewer the M <= 64 kernel is level with it); above 64 rows, while
-// there is at most one 32 x 32 tile a CU, the MFMA kernel (N=48: 2048 rows 32.6 -> 16.6 us; N=512,
+// there is at most one 32 x 32 tile a CU, the MFMA kernel (N=48: 2048 rows 32.6 -> 14.9 us; N=512,
 // 333 rows 22.3 -> 15.1; with two tiles a CU level with the tile kernel, behind it from there).
 constexpr int64_t kRowsDotOutputs = 16384, kRowsDotColumns = 1024;
 

@@ -123,3 +123,9 @@ def test_pair(rt, rows, n, k):
 @pytest.mark.parametrize("rows,n,k", [(3, 48, 1088), (2, 1024, 5120), (33, 48, 192), (5, 481, 320), (64, 96, 8256)])
 def test_row_major_few_outputs(rt, rows, n, k):
     check_weight(rt, n, k, rows, tiled=False)
+
+
+# The MFMA kernel for more rows: fewer groups than its 16 waves, even and odd numbers of groups a wave.
+@pytest.mark.parametrize("rows,n,k", [(70, 512, 192), (333, 96, 1024), (129, 129, 1088), (600, 48, 2112)])
+def test_row_major_more_rows(rt, rows, n, k):
+    check_weight(rt, n, k, rows, tiled=False)
