@@ -298,7 +298,8 @@ q4_rows_mma_kernel(RowsArgs args) {
 // lane-per-row kernel, 2.7 here; N=5120 17.7 -> 6.7; N=17408 27.9 -> 17.7; two rows of N=17408 41 ->
 // 26); up to kRowsDotOutputs outputs of at most kRowsDotColumns columns on the same kernel
 // (N=48: 16 rows 10.0 -> 3.0 us, 64 rows 12 -> 4.7, 333 rows 19 -> 12; N=512, 16 rows 12.2 -> 7.5;
-// at 16384 outputs and 64 rows or fewer the M <= 64 kernel is level with it); above 64 rows, while
+// at 16384 outputs and 64 rows or fewer the M <= 64 kernel is level with it); above 66 rows (65 and 66 are 64
+// and a call of one or two, whose weights enter the sums exactly; this kernel rounds them to bf16), while
 // there is at most one 32 x 32 tile a CU, the MFMA kernel (N=48: 2048 rows 32.6 -> 14.9 us; N=512,
 // 333 rows 22.3 -> 15.1; with two tiles a CU level with the tile kernel, behind it from there).
 constexpr int64_t kRowsDotOutputs = 16384, kRowsDotColumns = 1024;
@@ -311,7 +312,7 @@ bool rows_fit(int64_t rows, int64_t columns, int64_t inner, int64_t lda) {
     if (rows < 1 || inner % kGroup != 0 || columns > (1 << 30) || inner > (1 << 30)) return false;
     if (rows_dot(rows, columns)) return true;
     // (The activations are read through a buffer resource: 32-bit byte offsets.)
-    return rows > 64 && (rows + 31) / 32 * ((columns + 31) / 32) <= device_cus() &&
+    return rows > 66 && (rows + 31) / 32 * ((columns + 31) / 32) <= device_cus() &&
            (rows * lda + inner) * 2 < ((int64_t)1 << 32) - 256;
 }
 
