@@ -521,11 +521,14 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs &args) {
             const int g = ga + t < gb ? ga + t : gb - 1;
             return (uint32_t)__builtin_amdgcn_readfirstlane(g);
         };
+        // (Past the job every offset lies past the buffer: zeros, no traffic. Zero weights alone would make NaN of
+        // infinite activations. Units of four steps have no such step that is multiplied.)
         auto load_a = [&](int t, int buf) {
             const uint32_t g = clampg(t), at = kUnit == 1 ? g * 128u : (g >> 2) * 512u + (g & 3u) * 64u;
+            const uint32_t past = kUnit == 1 && ga + t >= gb ? 0xFFFFFFF0u : 0u;
 #pragma unroll
             for (int p = 0; p < kAPer; ++p)
-                buffer_load_lds16(a_rsrc, lds + buf * kSBuf + 8192 * p + 1024 * wave, a_src[p] + at);
+                buffer_load_lds16(a_rsrc, lds + buf * kSBuf + 8192 * p + 1024 * wave, (a_src[p] + at) | past);
         };
         // Group t's weights in register set t mod 2 (s: t mod kUnit; jobs start on a unit).
         auto load_codes = [&](int t, int set, int s) { wst.load(clampg(t), set, s); };

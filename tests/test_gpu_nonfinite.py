@@ -129,3 +129,32 @@ def test_row_major_few_outputs(rt, rows, n, k):
 @pytest.mark.parametrize("rows,n,k", [(70, 512, 192), (333, 96, 1024), (129, 129, 1088), (600, 48, 2112)])
 def test_row_major_more_rows(rt, rows, n, k):
     check_weight(rt, n, k, rows, tiled=False)
+
+
+# Prefill: whole tiles and cut ones whose jobs have odd numbers of groups, one and several weights.
+@pytest.mark.parametrize("rows,n,k", [(129, 384, 2112), (200, 640, 192), (333, 1152, 1088), (700, 1152, 320)])
+def test_prefill(rt, rows, n, k):
+    c, d = case(n, k), case(128, k)
+    for value, place in INF:
+        bits = activations(rows, k, value, place)
+        a, ref = bf16_tensor(bits), reference(bits, c.dense)
+        for ws in workspaces(rt, rows, n + 128, k):
+            check(rt.gemm(c.w_tiled, a, out_dtype=torch.float32, workspace=ws, kernel=rt.PREFILL), ref,
+                  f"prefill {rows} {n} {k} {value} {place}")
+            outs = rt.gemm_group([c.w_tiled, d.w_tiled], a, out_dtype=torch.float32, workspace=ws)
+            check(outs[0], ref, f"grouped prefill {rows} {n} {k} {value} {place}")
+            check(outs[1], reference(bits, d.dense), f"grouped prefill {rows} 128 {k} {value} {place}")
+
+
+@pytest.mark.parametrize("rows,k", [(129, 1280), (333, 2304)])
+def test_prefill_planes(rt, rows, k):
+    n = 384
+    native = oracle.q45k_random_native(n, k, seed=n)
+    dense = oracle.q45k_decode(native).reshape(n, k)
+    from qcheck import dev_u8
+    w = rt.q5k_repack(dev_u8(native), n, k)
+    for value, place in INF:
+        bits = activations(rows, k, value, place)
+        for ws in workspaces(rt, rows, n, k):
+            check(rt.gemm(w, bf16_tensor(bits), out_dtype=torch.float32, workspace=ws, kernel=rt.PREFILL),
+                  reference(bits, dense), f"prefill planes {rows} {k} {value} {place}")
