@@ -740,7 +740,7 @@ static int gguf_gemm(const splosh_q5k_weight *w_in, bool fifth, const uint16_t *
                             "aligned operands");
             const splosh::PrefillPlan plan =
                 splosh::plan_prefill(rows, w->rows, w->inner / kGroupSize, workspace ? workspace_bytes : 0,
-                                     splosh::kPrefillDecodePlanes);
+                                     splosh::kPrefillPlanes);
             return hip_status(splosh::launch_q5k_prefill(plan, *w, fifth, a, lda, out, ldc, out_dtype, residual, rows,
                                                          workspace, stream),
                               "q5k prefill launch");
@@ -884,7 +884,7 @@ static int gguf_native_gemm(int gguf_type, const uint8_t *native, int64_t rows, 
         return e ? (int64_t)atoll(e) : kGgufPrefillRows;
     }();
     const bool units = inner % 256 == 0;
-    const double decode = units ? splosh::kPrefillDecodeUnits : splosh::kPrefillDecodeNative;
+    const splosh::PrefillFormat format = units ? splosh::kPrefillUnits : splosh::kPrefillNative;
     const int base_type = gguf_type & 0xFF;
     const int64_t stream_max = base_type == 11 ? 6 : base_type == 20 ? 3 : 4;
     // (The rows past 64 of a call of two are exact up to stream_max of them: the prefill kernel from the next.)
@@ -898,7 +898,7 @@ static int gguf_native_gemm(int gguf_type, const uint8_t *native, int64_t rows, 
     if (prefill && m < prefill_rows) {
         const size_t need = ho.on() ? splosh_heads_workspace_bytes(m, rows, inner)
                                     : splosh::prefill_plan_bytes(splosh::plan_prefill(
-                                          m, rows, inner / kGroupSize, (size_t)-1, decode));
+                                          m, rows, inner / kGroupSize, (size_t)-1, format));
         prefill = need == 0 || (workspace && workspace_bytes >= need);
     }
     // 65..128 rows: two calls of at most 64 rows, as for q4. K17408 -> N5120, against the tiled
@@ -931,7 +931,7 @@ static int gguf_native_gemm(int gguf_type, const uint8_t *native, int64_t rows, 
     }
     if (prefill) {
         const splosh::PrefillPlan plan = splosh::plan_prefill(m, rows, inner / kGroupSize, workspace ? workspace_bytes : 0,
-                                                              decode);
+                                                              format);
         return hip_status(splosh::launch_gguf_prefill(plan, gguf_type, native, rows, inner, a, lda, out, ldc, out_dtype,
                                                       residual, m, workspace, stream),
                           "gguf prefill launch");

@@ -197,8 +197,9 @@ hipError_t launch_q4_tile(const TilePlan &plan, const splosh_q4_weight &w, const
                           const uint16_t *a, int64_t lda, void *out, int64_t ldc, int out_dtype, const void *residual,
                           int64_t rows, void *workspace, hipStream_t stream);
 
-// The prefill kernel for one tiled weight (prefill.hip): 256 x 256 tiles, two waves per SIMD,
-// weights dequantized once a workgroup into LDS; stream-K over a caller workspace of prefill_workspace_bytes().
+// The prefill kernel for one tiled weight (prefill.hip): tiles of 128 to 256 rows by 256 columns, two waves per
+// SIMD, weights dequantized once a workgroup into LDS; the remaining tiles are split over K in a caller workspace
+// of prefill_workspace_bytes().
 struct PrefillPlan {
     int fm;            // tile rows / 64 (2, 3 or 4)
     int mblocks;       // row blocks of 64 fm
@@ -206,7 +207,7 @@ struct PrefillPlan {
     int grid;
     int sk_grid;       // workgroups that share the other tiles
     int dp_tiles;      // tiles computed whole (a multiple of grid)
-    int64_t sk_units;  // (tile, group) pairs of the other tiles, split evenly over sk_grid
+    int64_t sk_units;  // (tile, group) pairs of the other tiles, split evenly over sk_grid (in whole units)
 };
 // The weights of a grouped call side by side (columns col[i] .. col[i + 1] - 1 are weight i's).
 struct PrefillGroup {
@@ -217,11 +218,21 @@ struct PrefillGroup {
     int64_t ldc[SPLOSH_MAX_GROUP];
 };
 bool prefill_fits(int64_t rows, int64_t columns, int64_t inner, int64_t lda, int64_t ldc);
-// `decode`: what the format adds to a step's time (us; measured at 256-row tiles: Q4_K and Q5_K 2.1 us a
-// step against 1.75, the native formats 2.0 to 2.3 in whole units of 256, else 2.4 to 3.2).
-constexpr double kPrefillDecodeQ4 = 0.0, kPrefillDecodePlanes = 0.35, kPrefillDecodeNative = 1.0, kPrefillDecodeUnits = 0.3;
+// What the planner knows of a format. decode: what it adds to a step's time (us; measured at 256-row tiles:
+// Q4_K and Q5_K 2.1 us a step against 1.75, the native formats 2.0 to 2.3 in whole units of 256, else 2.4 to
+// 3.2). partial: a megabyte of partials (us). unit: the 64-groups its kernel splits K at (groups is a
+// multiple of it).
+struct PrefillFormat {
+    double decode, partial;
+    int unit;
+};
+// (kPrefillUnits: the pair that came nearest to the fastest cut on 25 shapes of 65 to 1024 rows and K512 to
+// K17408, each cut of each timed: 1.4% off on average and 10% at most, against 4.4% and 14% for the cuts of
+// shares counted in single groups. IQ3_S at K1536 lost 4 to 5% by it.)
+constexpr PrefillFormat kPrefillQ4{0.0, 0.15, 1}, kPrefillPlanes{0.35, 0.15, 1}, kPrefillNative{1.0, 0.15, 1},
+    kPrefillUnits{0.2, 0.25, 4};
 PrefillPlan plan_prefill(int64_t rows, int64_t columns, int64_t groups, size_t workspace_bytes,
-                         double decode = kPrefillDecodeQ4);
+                         PrefillFormat format = kPrefillQ4);
 size_t prefill_workspace_bytes(int64_t rows, int64_t columns, int64_t groups);
 // The workspace a plan uses.
 size_t prefill_plan_bytes(const PrefillPlan &plan);

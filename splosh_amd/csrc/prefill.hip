@@ -753,9 +753,11 @@ static size_t prefill_sk_bytes(int grid, int fm) {
 //  * a step of a tile of 128, 192 or 256 rows takes 0.87, 1.18 or 1.37 us while at most about 60% of
 //    the CUs work, and 1.12, 1.45 or 1.8 with all of them (the shader clock falls under the load, so a
 //    round that leaves CUs idle loses little: 160 whole tiles of 80 steps, K5120 -> N5120 at 2048 rows,
-//    take 119 us, split over all 256 CUs 132). `decode` is what the format's decoding adds to a step;
+//    take 119 us, split over all 256 CUs 132). `decode` is what the format's decoding adds to a step; a format
+//    that splits K at units of several groups has its shares counted in those (149 rows of K2560 -> N7936, Q8_0
+//    blocks: 5 slices of two units a tile take 29.3 us, 8 of which six hold one unit and two hold two 32.8);
 //  * a call whose last tiles are split costs 8.5 us more for the finish pass's launch and the partials'
-//    round trip, and 0.15 us a megabyte of partials.
+//    round trip, and 0.15 us a megabyte of partials (PrefillFormat).
 // Whole rounds of tiles come first; the remaining tiles are left whole, cut into S slices each (S a
 // tile's workgroups, so that no workgroup meets two tiles), or split evenly over all CUs. Measured
 // against even splits of 256-row tiles (us): 333 rows K5120 -> N5120 53.9 -> 40.6 (128 rows, 4 slices),
@@ -768,7 +770,9 @@ static double prefill_step_us(int fm, double busy, double decode) {
     return kIdle[fm] + (kFull[fm] - kIdle[fm]) * x + decode;
 }
 
-PrefillPlan plan_prefill(int64_t rows, int64_t columns, int64_t groups, size_t workspace_bytes, double decode) {
+PrefillPlan plan_prefill(int64_t rows, int64_t columns, int64_t groups, size_t workspace_bytes, PrefillFormat format) {
+    const double decode = format.decode;
+    const int64_t units = groups / format.unit;  // of a tile
     const int cus = prefill_grid();
     PrefillPlan best = {};
     double best_us = 0.0;
@@ -782,7 +786,7 @@ PrefillPlan plan_prefill(int64_t rows, int64_t columns, int64_t groups, size_t w
         const double whole = full / cus * (double)groups * prefill_step_us(fm, 1.0, decode);
         // s = 0: the remaining tiles evenly over all CUs; 1: whole; more: slices a tile.
         for (int s = 0; s <= 16; ++s) {
-            if ((s != 1 && rem == 0) || (s > 1 && ((int64_t)rem * s > cus || s > groups))) continue;
+            if ((s != 1 && rem == 0) || (s > 1 && ((int64_t)rem * s > cus || s > units))) continue;
             p.grid = p.tiles < cus ? p.tiles : cus;
             p.dp_tiles = p.tiles;
             p.sk_units = 0;
@@ -793,13 +797,13 @@ PrefillPlan plan_prefill(int64_t rows, int64_t columns, int64_t groups, size_t w
             } else {
                 p.dp_tiles = full;
                 p.sk_units = (int64_t)rem * groups;
-                p.sk_grid = s == 0 ? cus : rem * s;
+                p.sk_grid = s == 0 ? (int)(rem * units < cus ? rem * units : cus) : rem * s;
                 p.grid = full > 0 ? cus : p.sk_grid;
                 if (prefill_sk_bytes(p.sk_grid, fm) > workspace_bytes) continue;  // no room for partials
                 const double parts = p.sk_grid + (s == 0 ? rem : 0);
-                us += (double)((p.sk_units + p.sk_grid - 1) / p.sk_grid) *
+                us += (double)((rem * units + p.sk_grid - 1) / p.sk_grid * format.unit) *
                           prefill_step_us(fm, (double)p.sk_grid / cus, decode) +
-                      8.5 + 0.15 * parts * tile_mb;
+                      8.5 + format.partial * parts * tile_mb;
             }
             if (best.fm == 0 || us < best_us) {
                 best = p;
@@ -816,8 +820,9 @@ size_t prefill_plan_bytes(const PrefillPlan &plan) {
 
 size_t prefill_workspace_bytes(int64_t rows, int64_t columns, int64_t groups) {
     size_t need = 0;
-    for (const double decode : {kPrefillDecodeQ4, kPrefillDecodePlanes, kPrefillDecodeNative, kPrefillDecodeUnits}) {
-        const size_t bytes = prefill_plan_bytes(plan_prefill(rows, columns, groups, (size_t)-1, decode));
+    for (const PrefillFormat format : {kPrefillQ4, kPrefillPlanes, kPrefillNative, kPrefillUnits}) {
+        if (groups % format.unit != 0) continue;
+        const size_t bytes = prefill_plan_bytes(plan_prefill(rows, columns, groups, (size_t)-1, format));
         need = need > bytes ? need : bytes;
     }
     return need;
