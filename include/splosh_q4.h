@@ -64,22 +64,27 @@ typedef enum splosh_dtype { SPLOSH_F32 = 0, SPLOSH_BF16 = 1 } splosh_dtype;
 /* Kernel choice (the reference selects kernels through SPLOSH_* environment variables,
  * Runtime/Engine.swift:380-440; here the caller names one, or AUTO picks by rows). */
 typedef enum splosh_kernel {
-    SPLOSH_KERNEL_AUTO = 0,     /* one or two rows of tiled weights whose staged activation rows fit
-                                   80 KB (K up to about 18700): STREAM; 3..16 rows of tiled weights,
-                                   and up to 32 where it wins (skinny.hip), the raw-code MFMA kernel
-                                   without a barrier in its loop; else up to 64: DEQUANT (a single weight of at least two
-                                   64-column bands a CU as the pair of its column halves); 65..128:
-                                   rows 0..63 and the rest as two calls of the above (without the
-                                   emit; PREFILL from 80 rows of tiled weights of 80 Mi elements,
-                                   given its scratch); more: PREFILL for tiled weights with lda % 8 == 0 and
-                                   ldc % 4 == 0, else TILE; SCALAR for operands no other kernel
-                                   takes. A row-major weight of one or two rows, or of few outputs
-                                   (rows.hip), takes a latency-shaped kernel of its own first */
+    SPLOSH_KERNEL_AUTO = 0,     /* by layout, rows and size.
+                                   TILED128: 1-2 rows STREAM (their staged activations fit 80 KB, K
+                                   up to about 18700); 3-16 rows, and 17-32 where it is the faster,
+                                   the raw-code MFMA kernel (skinny.hip); else up to 64 DEQUANT (a
+                                   wide single weight as the pair of its column halves); 65-128 two
+                                   calls of those, or PREFILL from 80 rows of a weight of 80 Mi
+                                   elements given its scratch, or with the emit TILE or PREFILL;
+                                   more PREFILL (lda % 8 == 0, ldc % 4 == 0, 16-byte aligned
+                                   output), else TILE.
+                                   ROW_MAJOR: 1-2 rows or few outputs the kernels of rows.hip (the
+                                   pair and the emit: STREAM at 1-2 rows); else up to 64 DEQUANT,
+                                   65-128 two calls, more TILE.
+                                   Operands that none of these takes: STREAM or SCALAR. */
     SPLOSH_KERNEL_STREAM = 1,   /* weight streaming on raw codes: the every-CU decode kernel for
                                    1-4 rows of tiled weights (with a workspace it splits the last
                                    round of row blocks over K, so every CU gets the same share),
                                    the lane-per-row kernel for row-major ones, the raw-code MFMA
-                                   kernel for more rows */
+                                   kernel for more rows. On raw codes an infinite activation or
+                                   scale makes NaN of a row's or output's sums (the kernels AUTO
+                                   takes from three rows, and for a group from one, give the
+                                   infinities of the dequantized weights) */
     SPLOSH_KERNEL_DEQUANT = 2,  /* rows <= 64: stream-K MFMA kernel on weights dequantized to bf16 in
                                    registers; uses the workspace for split bands when given one */
     SPLOSH_KERNEL_TILE = 3,     /* any rows: LDS-tiled dequant-to-bf16 MFMA GEMM (prefill) */
@@ -206,10 +211,12 @@ int splosh_q4_gemm_noalloc(const splosh_q4_weight *w, const uint16_t *a, int64_t
  * concurrent encoder so that they overlap (Runtime/Engine.swift:1402, SploshCore/CommandGraph.swift:
  * 57-62; the GEMMs at Engine.swift:1131-1140). out_i = a @ dequant(w_i)^T for i < count
  * (count <= SPLOSH_MAX_GROUP), each into its own output (row stride ldcs[i], out_dtype), no
- * residual. All weights share inner. Up to 64 rows with TILED128 weights (rows % 64 == 0) the
- * group is one launch of the M <= 64 kernel (at few rows the one AUTO gives a single weight from
- * three rows) over the weights' joined column bands, split over the CUs as one call (workspace: splosh_workspace_bytes(rows, sum of the weights' rows, inner));
- * otherwise each weight is its own splosh_q4_gemm call, same results to the path's tolerance. */
+ * residual. All weights share inner. TILED128 weights run side by side as one weight of their joined
+ * columns: up to 64 rows one launch of the M <= 64 kernel (at few rows of the one AUTO gives a single
+ * weight from three rows), 65..128 rows under AUTO two such calls, more one launch of the prefill kernel
+ * (ldcs[i] % 4 == 0, 16-byte aligned outputs). At every row count they split K in a workspace of
+ * splosh_workspace_bytes(rows, sum of the weights' rows, inner); a smaller one leaves work unsplit.
+ * Otherwise each weight is its own splosh_q4_gemm call, same results to the path's tolerance. */
 #define SPLOSH_MAX_GROUP 8
 int splosh_q4_gemm_group(const splosh_q4_weight *weights, int count, const uint16_t *a, int64_t lda,
                          void *const *outs, const int64_t *ldcs, int out_dtype, int64_t rows, int kernel,
@@ -246,12 +253,12 @@ int splosh_untile128(const void *src, void *dst, int64_t rows, int64_t groups, i
 
 /* Engine.gemm on a GGUF weight (Runtime/Engine.swift:1671-1697, kernels
  * Shaders/engine_gguf.metal:82-221 instantiated _q5k at :332-349). AUTO: one row takes the
- * every-CU decode kernel; 2..64 rows the dequant-to-bf16 MFMA kernel (DEQUANT; lda % 8 == 0 and
- * 16-byte aligned activations), 65..128 rows two calls of at most 64; more rows the 256-column
- * prefill kernel (PREFILL; also ldc % 4 == 0
- * and 16-byte aligned outputs), else the LDS-tiled kernel (TILE), else the streaming kernel
- * (STREAM). DEQUANT and PREFILL use a workspace of splosh_workspace_bytes(rows, w->rows, w->inner)
- * to split K. Odd alignments fall back to SCALAR. */
+ * every-CU decode kernel; 5..16 rows (2..4 of the larger weights) the barrier-free MFMA kernel of
+ * skinny_gguf.hip, else up to 64 rows the stream-K one (DEQUANT), both on weights dequantized to bf16
+ * (lda % 8 == 0 and 16-byte aligned activations); 65..128 rows two calls of at most 64; more rows the
+ * prefill kernel (PREFILL; also ldc % 4 == 0 and 16-byte aligned outputs), else the LDS-tiled kernel
+ * (TILE), else the streaming kernel (STREAM). The MFMA kernels use a workspace of
+ * splosh_workspace_bytes(rows, w->rows, w->inner) to split K. Odd alignments fall back to SCALAR. */
 int splosh_q5k_gemm(const splosh_q5k_weight *w, const uint16_t *a, int64_t lda, void *out, int64_t ldc,
                     int out_dtype, const void *residual, int64_t rows, int kernel, void *workspace,
                     size_t workspace_bytes, hipStream_t stream);

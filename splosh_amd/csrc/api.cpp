@@ -89,8 +89,12 @@ bool q4_stream_eligible(const splosh_q4_weight &w, const uint16_t *a, int64_t ld
 // 80..128 rows of a weight this large (elements): one call of the prefill kernel (128-row tiles) instead of
 // two of at most 64 rows, given its scratch. Two calls / one (us): K5120 -> N17408 at 65 rows 42.9 / 46.1, 80
 // 44.4 / 43.6, 96 49.6 / 44.1, 128 54.4 / 45.2; its gate+up 67.5 / 69.6, 69.3 / 66.5, 75.4 / 67.8, 85.9 / 74.1;
-// K17408 -> N5120 41.0 / 44.4, 49.6 / 43.1, 46.8 / 43.6, 52.1 / 44.1. Not the smaller ones: K5120 -> N12288 at
-// 96 rows 32.9 / 34.8, N5120 25.7 / 27.7.
+// K17408 -> N5120 41.0 / 44.4, 49.6 / 43.1, 46.8 / 43.6, 52.1 / 44.1; K8192 -> N10240 (80 Mi) 37.4 / 39.7, 41.1 /
+// 41.1, 46.8 / 42.7, 51.5 / 45.2. Below the line two calls are mostly the faster: K5120 -> N15360 (75 Mi) at 128
+// rows 37.1 / 40.5, K8192 -> N8192 40.4 / 40.5, K5120 -> N12288 at 96 rows 32.9 / 34.8. Size alone does not settle
+// it: K14336 -> N5120 (70 Mi) at 96 and 128 rows 41.1 / 40.1 and 45.4 / 40.9, and the pair, of which one weight is
+// counted, of 2 x N10240 at K5120 (50 Mi each) 57 / 43.5 and 62 / 45, but of 2 x N12288 54 / 53 and 54 / 55, of
+// 2 x N14336 at K4096 49 / 51 and 50 / 50.
 constexpr int64_t kPrefillLargeWeight = 80 << 20, kPrefillLargeRows = 80;
 
 int q4_gemm_impl(const splosh_q4_weight *w, const splosh_q4_weight *up, const uint16_t *a, int64_t lda, void *out,
@@ -160,9 +164,11 @@ int q4_gemm_impl(const splosh_q4_weight *w, const splosh_q4_weight *up, const ui
         else if (wide16 && splosh::lanes_fit(rows, w->rows, w->inner, w->row_stride_words, up != nullptr))
             choice = SPLOSH_KERNEL_STREAM;
         else if (mma_ok) choice = SPLOSH_KERNEL_DEQUANT;
-        // One weight at 65..128 rows: the tile kernel where the prefill kernel's 256-row tiles are
-        // mostly padding and its tiles few (measured at M=64..128: K17408 -> N5120 tile 51-56 us,
-        // prefill 59-65; K5120 -> N17408 tile better at 65 rows, prefill from 96).
+        // One weight at 65..128 rows that none of the routes above took, as a call with the emit: the tile
+        // kernel and the operand pass up to 80 rows or 8192 outputs, a line drawn when the prefill kernel had
+        // tiles of 256 rows only. With its tiles of 128 rows and its fused emit the prefill kernel is the faster
+        // (residual and emit, this route / PREFILL by name at 65, 96 and 128 rows, us: K17408 -> N5120 54.5 /
+        // 43.6, 53.0 / 42.4, 57.3 / 44.1; K5120 -> N5120 29.0 / 25.4, 29.6 / 27.0, 32.6 / 29.5).
         else if (tile_ok && !up && rows <= 128 && (rows <= 80 || w->rows <= 8192)) choice = SPLOSH_KERNEL_TILE;
         else if (prefill_ok || prefill_mlp_ok) choice = SPLOSH_KERNEL_PREFILL;
         else if (tile_ok) choice = SPLOSH_KERNEL_TILE;
@@ -684,8 +690,10 @@ static int gguf_gemm(const splosh_q5k_weight *w_in, bool fifth, const uint16_t *
     const splosh_q5k_weight *w = &wv;
     if ((st = check_io(a, lda, out, ldc, out_dtype, rows, w->rows, w->inner))) return st;
     const bool planes_ok = aligned(w->plane0, 16) && (!fifth || aligned(w->plane1, 4)) && aligned(w->meta, 16);
-    // 65..128 rows under AUTO: two calls of at most 64 rows, as for q4 (K17408 -> N5120, against the
-    // prefill kernel: M=96 66 -> 54 us, M=128 69 -> 59).
+    // 65..128 rows under AUTO: two calls of at most 64 rows, as for q4, a line drawn when the prefill kernel
+    // had tiles of 256 rows only (K17408 -> N5120 at 96 and 128 rows 66 and 69 us). Two calls / PREFILL by name
+    // with its tiles of 128 rows, at 65, 80, 96 and 128 rows (Q5_K, us): K17408 -> N5120 49.4 / 46.4, 53.5 /
+    // 44.7, 53.8 / 45.1, 58.7 / 47.2; K5120 -> N17408 44.2 / 46.1, 50.5 / 47.6, 53.5 / 48.9, 59.2 / 52.2.
     if (kernel == SPLOSH_KERNEL_AUTO && rows > 64 && rows <= 128 && planes_ok && lda % 8 == 0 && aligned(a, 16) &&
         splosh::q5k_mma_fits(64, w->rows, w->inner, lda)) {
         const char *res = (const char *)residual;

@@ -422,8 +422,9 @@ struct GgufStage {
 // step, and those of a super-block overlap (Q6_K: eight loads a thread and step, each lane in a cache line
 // of its own, the step bound by them). K5120 -> N17408, 1024 rows, ROWS32: Q6_K 250 -> 205 us, Q3_K 237 ->
 // 191, IQ3_S 289 -> 205, IQ4_XS 207 -> 190, Q8_0 216 -> 202, IQ4_NL 201 -> 190. The Q4_K and Q5_K planes, whose
-// records are coalesced as they are, gain nothing from it. At 256 rows a few of the unit's registers spill in the
-// loop; loading Q6_K's low nibbles in two parts halved that and changed nothing.
+// records are coalesced as they are, gain nothing from it. At 256 rows the loop spills registers (VGPRs: Q6_K 39,
+// Q3_K 30, Q8_0 24, IQ3_S 14, IQ4_NL 11, IQ4_XS 10; at 192 rows two of Q8_0, at 128 none); loading Q6_K's low
+// nibbles in two parts halved its spills and changed no time.
 template <int TYPE>
 struct GgufUnitStage {
     static constexpr int kLoads = 0, kNW = 1, kUnit = 4, kTbl = Half<TYPE>::kTbl;
@@ -646,7 +647,8 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs &args) {
     }
 }
 
-// 256-row tiles of one weight or the fused pair; lower tiles and grouped weights.
+// 256-row tiles of the stages marked kTall; every other tile. (The bodies are the same: the two names part the
+// ten 256-row kernels that tests/test_mma_waitcounts.py counts from those of tests/test_prefill_tiles.py.)
 template <class W>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 prefill_kernel(PrefillArgs args) {
