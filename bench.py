@@ -40,10 +40,12 @@ MEASURED_TRAFFIC = {
     ("lmhead1", "lm_head"): 349321.9 * 2 * 1024 + 526.2 * 1024,  # q4_decode_kernel<1, 1, 32, 2>
     ("q5k1", "q5k"): 30124.4 * 2 * 1024 + 30.0 * 1024,  # q5k_decode_kernel<8, 2, true>
     ("q5k64", "q5k"): 41299.7 * 2 * 1024 + 4303.0 * 1024,  # mma_kernel<Q5Format<2, 4, 3, true>, 2, 2, 4, 3>
-    ("q5k16", "q5k"): 32869.4 * 2 * 1024 + 1050.0 * 1024,  # mma_kernel<Q5Format<2, 4, 3, true>, 1, 2, 4, 3>
-    ("prefill2048", "prefill_up"): 264791.5 * 2 * 1024 + 114688.0 * 1024,  # prefill_kernel<Q4Stage>
-    ("q5k2048", "q5k"): 347729.4 * 2 * 1024 + 98304.0 * 1024,  # prefill_kernel<Q5Stage<true>>
-    ("q6k2048", "gguf"): 366940.1 * 2 * 1024 + 110080.0 * 1024,  # prefill_kernel<GgufStage<14>>
+    ("q5k16", "q5k"): 32666.8 * 2 * 1024 + 1140.0 * 1024,  # gguf_skinny_kernel<13, 16>
+    ("prefill2048", "prefill_up"): 266503.5 * 2 * 1024 + 114688.0 * 1024,  # prefill_kernel<Q4Stage>
+    ("q5k2048", "q5k"): 343039.9 * 2 * 1024 + 98304.0 * 1024,  # prefill_kernel<Q5Stage<true>>
+    ("q6k2048", "gguf"): 379349.1 * 2 * 1024 + 118272.0 * 1024,  # prefill_kernel<GgufUnitStage<14>>
+    ("q6k8", "gguf"): 38046.6 * 2 * 1024 + 580.0 * 1024,  # gguf_skinny_kernel<14, 8>
+    ("q6k24", "gguf"): 41101.6 * 2 * 1024 + 2180.0 * 1024,  # gguf_skinny_kernel<14, 32>
     ("q6k64", "gguf"): 47875.7 * 2 * 1024 + 4212.1 * 1024,  # mma_kernel<GgufFormat<14, 2, 4, 3>, 2, 2, 4, 3>
     ("iq3s64", "gguf"): 30858.2 * 2 * 1024 + 4174.7 * 1024,  # mma_kernel<GgufFormat<21, 2, 4, 3>, 2, 2, 4, 3>
     ("q6k64r", "gguf"): 47010.9 * 2 * 1024 + 4340.4 * 1024,  # the same, Q6_K in the ROWS32 order
