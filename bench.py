@@ -1,6 +1,6 @@
 """Benchmark of the quantized-matmul hot path on one MI355X.
 
-Default workload (the draft-verify step the metric is quoted on): M = 64
+Default workload (the draft-verify step): M = 64
 activation rows (8 sessions x 8 drafted tokens), 4-bit g64 affine weights, the fused gate+up
 projection (two K=5120 -> N=17408 weights sharing one activation read, out = silu(g) * u) followed
 by the down projection (K=17408 -> N=5120) on that output. One "step" is that pair of launches.
@@ -180,8 +180,8 @@ def build_workload(name, rt, torch, gen, kernel):
                "weight_copies": ncopy}
         return launches, b, 2 * m * n * k, {"gemv": b}, cfg, {"gemv": 2 * m * n * k}
     if name == "layerset":
-        # Config 4: every linear projection of one hybrid layer set at M=64 (shapes as BASELINE.json
-        # states them): attention q, k, v, o; gated-delta input (qkv+z+b/a, 12288 outputs) and
+        # Config 4: every linear projection of one hybrid layer set at M=64 (the reference's model):
+        # attention q, k, v, o; gated-delta input (qkv+z+b/a, 12288 outputs) and
         # output (6144 -> 5120); the MLP's fused gate+up and down. The attention layer's q, k and v
         # read one activation and go as one grouped launch (splosh_q4_gemm_group, the reference's
         # concurrent encoder); one step is six launches over the nine weights.

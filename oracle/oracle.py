@@ -301,7 +301,7 @@ def q45k_gemm_native(a_bf16, native, N, K, fifth_bit=True, n0=0, n1=None, thread
     return out
 
 
-# ---- seeded synthetic inputs (the BASELINE distributions) -----------------------------------
+# ---- seeded synthetic inputs (the benchmark's distributions) -----------------------------------
 
 def q4_random_weight(N, K, seed, stride_words=None):
     """Row-major padded MLX q4 weight: uniform random code words, scale = bf16(|N(0, 0.02)|),

@@ -54,7 +54,7 @@ class Q4Case:
 
 
 def check_close(got, ref, *, bf16_out, tight=False, absref=None, label=""):
-    """The path's tolerance (BASELINE north_star): max |err| / max |ref| <= 1e-2 and cosine >=
+    """The path's tolerance: max |err| / max |ref| <= 1e-2 and cosine >=
     0.9999 against the fp32-accumulate reference, plus the reference tests' sum-normalised relErr
     <= 1e-2 (GemmOracleTests.swift:155-158).
 

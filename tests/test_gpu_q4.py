@@ -235,7 +235,7 @@ def test_workspace_shared_by_prefill_and_split_k(rt):
 
 
 def _full_size_weight(rt, n, k, seed):
-    """A BASELINE-size tiled q4 weight generated on the device (uniform code words,
+    """A full-size tiled q4 weight generated on the device (uniform code words,
     scale = bf16(|N(0, 0.02)|), bias = bf16(N(0, 0.01)))."""
     gen = torch.Generator(device="cuda").manual_seed(seed)
     groups = k // 64
