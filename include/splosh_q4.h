@@ -82,11 +82,13 @@ typedef enum splosh_kernel {
                                    round of row blocks over K, so every CU gets the same share),
                                    the lane-per-row kernel for row-major ones, the raw-code MFMA
                                    kernel for more rows. On raw codes an infinite activation or
-                                   scale makes NaN of a row's or output's sums (the kernels AUTO
-                                   takes from three rows, and for a group from one, give the
-                                   infinities of the dequantized weights) */
+                                   scale makes NaN of a row's or output's sums (the few-row kernels
+                                   of AUTO and PREFILL give the infinities of the dequantized
+                                   weights) */
     SPLOSH_KERNEL_DEQUANT = 2,  /* rows <= 64: stream-K MFMA kernel on weights dequantized to bf16 in
-                                   registers; uses the workspace for split bands when given one */
+                                   registers; uses the workspace for split bands when given one. A
+                                   row with an infinite activation can be NaN where its step is
+                                   partly idle, in place of infinities */
     SPLOSH_KERNEL_TILE = 3,     /* any rows: LDS-tiled dequant-to-bf16 MFMA GEMM (prefill) */
     SPLOSH_KERNEL_SCALAR = 4,   /* one thread per output (gemm_q4.metal semantics) */
     SPLOSH_KERNEL_PREFILL = 5   /* TILED128 q4 weights (mlp_in: 128 columns of each a tile,
