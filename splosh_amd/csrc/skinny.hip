@@ -311,19 +311,26 @@ static int skinny_rows(int64_t rows) { return rows <= 8 ? 8 : rows <= 16 ? 16 : 
 //  * for fewer blocks than CUs and long K (24 groups a wave), two workgroups a CU (K17408 -> N5120:
 //    18.9 -> 17.3 us): the merge costs about 3 us, which shorter K does not win back (K5120 -> N5120
 //    8.2 -> 9.8).
+// The registers of two weights and 32 rows leave a CU one workgroup of eight waves or three of four. So the pair
+// takes four waves from a block a CU (a second round of eight-wave workgroups would find most CUs empty: 24 rows of
+// K4096 -> 2 x N12288 21.6 -> 19.6 us, of K1536 13.9 -> 10.4; 16 rows of K5120 21.3 -> 20.0, at 8 rows level), and its
+// slices of 17 to 32 rows are planned for one workgroup a CU (K17408 -> 2 x N4096, 24 rows 33.8 -> 26.5 us; the
+// stream-K kernel 27.8). At 32 rows that kernel is still up to 17% faster where its bands come out whole (K5120 -> 2 x
+// N12288 26.0 here, 23.6), on weights rounded to bf16.
 constexpr int kSkinnyLong = 24;
 struct SkinnyPlan {
     int kw;
     BalanceSplit split;
 };
-static SkinnyPlan plan_skinny(int64_t blocks, int groups) {
+static SkinnyPlan plan_skinny(int64_t blocks, int groups, int64_t rows, int nw) {
     SkinnyPlan p;
     const int cus = device_cus();
-    p.kw = blocks >= 2 * cus ? 4 : 8;
+    p.kw = blocks >= 2 * cus || (nw == 2 && rows > 8 && blocks > cus) ? 4 : 8;
     p.split = plan_balance(blocks, cus, groups);
+    const int per_cu = groups < kSkinnyLong * p.kw || (nw == 2 && rows > 16) ? 1 : 2;
     int s = 1;
-    if (2 * blocks <= cus) s = (int)(cus / blocks) * (groups >= kSkinnyLong * p.kw ? 2 : 1);
-    else if (blocks < cus && groups >= kSkinnyLong * p.kw) s = (int)(2 * cus / blocks);
+    if (2 * blocks <= cus) s = (int)(cus / blocks) * per_cu;
+    else if (blocks < cus && per_cu == 2) s = (int)(2 * cus / blocks);
     s = s < kBalanceMaxSlices ? s : kBalanceMaxSlices;
     while (s >= 2 && (groups < 2 * s * p.kw || blocks * s % 8 != 0)) --s;
     if (s >= 2) p.split = BalanceSplit{0, (int)blocks, s};
@@ -366,9 +373,11 @@ static size_t skinny_need(const SkinnyPlan &p, int64_t rows, int nw) {
 size_t skinny_workspace_bytes(int64_t rows, int64_t columns, int64_t inner, int nw) {
     if (!skinny_fits(rows, columns, inner, inner, nw == 2)) return 0;
     const int groups = (int)(inner / kGroup);
-    const size_t need = skinny_need(plan_skinny(columns / kSkinnyCols, groups), rows, nw);
+    size_t need = skinny_need(plan_skinny(columns / kSkinnyCols, groups, rows, 1), rows, 1);
+    const size_t pair = nw == 2 ? skinny_need(plan_skinny(columns / kSkinnyCols, groups, rows, 2), rows, 2) : 0;
+    need = need > pair ? need : pair;
     if (!skinny_split(columns, groups)) return need;
-    const size_t split = skinny_need(plan_skinny(columns / (2 * kSkinnyCols), groups), rows, 2);
+    const size_t split = skinny_need(plan_skinny(columns / (2 * kSkinnyCols), groups, rows, 2), rows, 2);
     return need > split ? need : split;
 }
 
@@ -403,7 +412,7 @@ template <SkinnyMode MODE>
 static hipError_t launch_skinny(SkinnyArgs &args, int64_t blocks, int64_t rows, void *workspace, size_t workspace_bytes,
                                 hipStream_t stream) {
     const int rm = skinny_rows(rows);
-    const SkinnyPlan p = plan_skinny(blocks, args.groups);
+    const SkinnyPlan p = plan_skinny(blocks, args.groups, rows, skinny_nw(MODE));
     const size_t need = skinny_need(p, rows, skinny_nw(MODE));
     args.slices = 1;
     if (need > 0 && workspace && workspace_bytes >= need) {
