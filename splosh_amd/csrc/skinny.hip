@@ -14,14 +14,15 @@
 //    its own, eight rows a load, and are read back as MFMA operands; codes and sidecars go to a
 //    register ring. All of a group's loads are issued D groups before its arithmetic and waited
 //    for with a counted vmcnt: no wave waits for another before the end.
-//  * Raw codes: a code word becomes four bf16 pairs (16 + q_j, 16 + q_{j+4}) with a shift and a
-//    v_and_or_b32 each, and the activation pairs are permuted to match ((x_j, x_{j+4}), shared by both
-//    weights). Per group, P = sum x (16 + q) and the row sums S = sum x (the same operands times ones,
-//    one chain for both weights) come from the matrix cores, and acc += s P + (b - 16 s) S takes two
+//  * Raw codes: a code word becomes four bf16 pairs (128 + q_j, 128 + q_{j+4}) with one v_and_or_b32
+//    each, and the activation pairs are permuted to match ((x_j, x_{j+4}), shared by both weights).
+//    Per group, P = sum x (128 + q) and the row sums S = sum x (the same operands times ones, one
+//    chain for both weights) come from the matrix cores, and acc += s P + (b - 128 s) S takes two
 //    FMAs a value: the weights are exact, where rounding them to bf16 in registers takes 19
-//    instructions per 8 weights (8 here). (128 + q saves a shift a word, but P and S cancel to a
-//    thirtieth there, and the fp32 sums came out further from 64 bits than the decode kernel's.) The cost of the scaling grows with the rows; at 64 the
-//    two are equal.
+//    instructions per 8 weights (7 here). The cost of the scaling grows with the rows; at 64 the
+//    two are equal. P and S cancel to a thirtieth, which left the fp32 sums of three and four rows further
+//    from 64 bits than the decode kernel's: calls of up to eight rows, but for grouped ones, use 16 + q, a shift
+//    more a word (1 to 3% of the time).
 //  * At the end the waves' sums meet in LDS in wave order. Where the blocks do not fill the CUs
 //    evenly, or are few, K is cut into slices merged by the last to arrive in slice order
 //    (balance_merge, common.hpp).
@@ -95,6 +96,8 @@ q4_skinny_kernel(SkinnyArgs args) {
     constexpr int NW = skinny_nw(MODE);
     using S = SkinnyShape<RM, KW, D>;
     constexpr int E = S::kE, NA = RM / 8;
+    constexpr bool kNear = RM == 8 && MODE != kSkinnyGroup;  // codes as 16 + q, else 128 + q
+    constexpr float kOffset = kNear ? 16.0f : 128.0f;
     constexpr int kLoads = 3 * NW + NA;  // loads a wave and group
     static_assert((D - 1) * kLoads <= 63, "vmcnt holds 6 bits");
     extern __shared__ __align__(16) char lds[];
@@ -163,9 +166,10 @@ q4_skinny_kernel(SkinnyArgs args) {
 #pragma unroll
     for (int k = 0; k < D; ++k) issue(k, k);
 
-    const uint32_t kMask = 0x00780078u;
-    uint32_t magic;  // the bf16 exponent of 16 in both halves: q in bits 3 .. 6 adds q
-    asm volatile("v_mov_b32 %0, 0x41804180" : "=v"(magic));
+    const uint32_t kMask = kNear ? 0x00780078u : 0x000F000Fu;
+    uint32_t magic;  // the bf16 exponent of 16 (q in bits 3 .. 6 adds q) or 128 (bits 0 .. 3) in both halves
+    if constexpr (kNear) asm volatile("v_mov_b32 %0, 0x41804180" : "=v"(magic));
+    else asm volatile("v_mov_b32 %0, 0x43004300" : "=v"(magic));
     const u32x4 ones = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};
     f32x16 zero;
 #pragma unroll
@@ -199,8 +203,9 @@ q4_skinny_kernel(SkinnyArgs args) {
 #pragma unroll
                 for (int w = 0; w < NW; ++w) {
                     const uint32_t q = cq[k][w][i];
-                    const u32x4 b = {sk_and_or(q << 3, kMask, magic), sk_and_or(q >> 1, kMask, magic),
-                                     sk_and_or(q >> 5, kMask, magic), sk_and_or(q >> 9, kMask, magic)};
+                    constexpr int kUp = kNear ? 3 : 0;
+                    const u32x4 b = {sk_and_or(q << kUp, kMask, magic), sk_and_or(q >> (4 - kUp), kMask, magic),
+                                     sk_and_or(q >> (8 - kUp), kMask, magic), sk_and_or(q >> (12 - kUp), kMask, magic)};
                     prod[w] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x[i], as_bf16x8(b), prod[w], 0, 0, 0);
                 }
                 // (Keeps the second half's operands from being built early: 28 bytes a lane spilled at 8 rows.)
@@ -209,7 +214,7 @@ q4_skinny_kernel(SkinnyArgs args) {
 #pragma unroll
             for (int w = 0; w < NW; ++w) {
                 const float s = bf16_bits_to_f32(cs[k][w]);
-                const float bp = __builtin_fmaf(-16.0f, s, bf16_bits_to_f32(cb[k][w]));
+                const float bp = __builtin_fmaf(-kOffset, s, bf16_bits_to_f32(cb[k][w]));
 #pragma unroll
                 for (int e = 0; e < E; ++e)
                     acc[w][e] = __builtin_fmaf(s, prod[w][e], __builtin_fmaf(bp, sum[e], acc[w][e]));
@@ -231,7 +236,7 @@ q4_skinny_kernel(SkinnyArgs args) {
     for (int w = 0; w < NW; ++w)
 #pragma unroll
         for (int e = 0; e < E; ++e) red[((wave * NW + w) * E + e) * 64 + lane] = acc[w][e];
-    // An infinite activation or scale leaves inf - inf in s P + (b - 16 s) S, and one above 2^123 can overflow
+    // An infinite activation or scale leaves inf - inf in s P + (b - 128 s) S, and one above 2^120 can overflow
     // it where x w does not: a wave with such a sum goes over its groups again with the dequantized weights (as
     // mma.hip) and takes the new sums in the place of those. No finite sum changes. (Here, with the sums in LDS,
     // it costs a call without such values less than 1%; before they leave the registers 1 to 5%.)
