@@ -311,8 +311,10 @@ static int skinny_rows(int64_t rows) { return rows <= 8 ? 8 : rows <= 16 ? 16 : 
 // each). Four waves where every CU gets at least two workgroups, else eight (K5120 -> N5120, 160
 // blocks, 8 rows: 9.8 us at four waves, 7.8 at eight; gate+up, 544 blocks: 22 and 24.7). K is sliced
 //  * for the last round of many blocks (plan_balance);
-//  * for at most half a block a CU, one workgroup a CU (K5120 -> N1024: 6.6 -> 5.8 us in 8 slices
-//    of 32 blocks);
+//  * for at most half a block a CU, one workgroup a CU, from K4096 (where a block gets fewer than four slices from
+//    K4608, or K5120 at one weight of up to four rows): four rows of K5120 -> N1024 6.8 -> 6.0 us in 5 slices, K4096
+//    -> N1024 6.0 -> 5.75 in 4, but K4096 -> N2560 6.2 -> 7.0 in 3, K3072 -> N1024 5.2 -> 5.5 in 3, K2048 4.4 -> 5.2
+//    in 2; 16 rows of the pair of K4608 -> 2 x N2560 10.7 -> 9.95 in 3;
 //  * for fewer blocks than CUs and long K (24 groups a wave), two workgroups a CU (K17408 -> N5120:
 //    18.9 -> 17.3 us): the merge costs about 3 us, which shorter K does not win back (K5120 -> N5120
 //    8.2 -> 9.8).
@@ -334,7 +336,8 @@ static SkinnyPlan plan_skinny(int64_t blocks, int groups, int64_t rows, int nw) 
     p.split = plan_balance(blocks, cus, groups);
     const int per_cu = groups < kSkinnyLong * p.kw || (nw == 2 && rows > 16) ? 1 : 2;
     int s = 1;
-    if (2 * blocks <= cus) s = (int)(cus / blocks) * per_cu;
+    const int least = 4 * blocks <= cus ? 64 : nw == 1 && rows <= 4 ? 80 : 72;
+    if (2 * blocks <= cus) s = groups < least ? 1 : (int)(cus / blocks) * per_cu;
     else if (blocks < cus && per_cu == 2) s = (int)(2 * cus / blocks);
     s = s < kBalanceMaxSlices ? s : kBalanceMaxSlices;
     while (s >= 2 && (groups < 2 * s * p.kw || blocks * s % 8 != 0)) --s;
