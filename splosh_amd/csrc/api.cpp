@@ -141,10 +141,11 @@ int q4_gemm_impl(const splosh_q4_weight *w, const splosh_q4_weight *up, const ui
                             res ? res + 64 * ldc * esize : nullptr, rows - 64, kernel, workspace, workspace_bytes,
                             stream);
     }
-    // 3..32 rows of tiled weights (one and two rows: the decode kernel below, unless their staged
-    // activations do not fit it).
+    // 3..32 rows of tiled weights (one and two rows, and a few shapes of three and four: the decode kernel
+    // below, unless their staged activations do not fit it).
     if (kernel == SPLOSH_KERNEL_AUTO && wide16 && w->order == SPLOSH_Q4_TILED128 &&
-        (rows >= 3 || !splosh::decode_fits(rows, w->rows, w->inner, w->order)) &&
+        !(splosh::decode_before_skinny(rows, w->rows, w->inner, up != nullptr) &&
+          splosh::decode_fits(rows, w->rows, w->inner, w->order)) &&
         splosh::skinny_fits(rows, w->rows, w->inner, lda, up != nullptr))
         return hip_status(splosh::launch_q4_skinny(*w, up, a, lda, out, ldc, out_dtype, residual, rows, workspace,
                                                    workspace ? workspace_bytes : 0, stream),
@@ -452,7 +453,8 @@ size_t splosh_workspace_bytes(int64_t rows, int64_t columns, int64_t inner) {
 size_t splosh_q4_workspace_bytes(const splosh_q4_weight *w, int64_t lda, int64_t rows, int pair) {
     if (!w || rows <= 0 || w->rows <= 0 || w->inner < kGroupSize) return 0;
     if (w->order == SPLOSH_Q4_TILED128) {
-        if (rows <= 2 && splosh::decode_fits(rows, w->rows, w->inner, w->order))
+        if (splosh::decode_before_skinny(rows, w->rows, w->inner, pair != 0) &&
+            splosh::decode_fits(rows, w->rows, w->inner, w->order))
             return splosh::decode_workspace_bytes(rows, w->rows, w->inner, pair ? 2 : 1);
         if (splosh::skinny_fits(rows, w->rows, w->inner, lda, pair != 0))
             return splosh::skinny_workspace_bytes(rows, w->rows, w->inner, pair ? 2 : 1);

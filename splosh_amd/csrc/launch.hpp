@@ -74,6 +74,8 @@ hipError_t launch_q4_decode(const splosh_q4_weight &w, const splosh_q4_weight *u
 // workgroup, no barrier in its loop. With a workspace of skinny_workspace_bytes (zero: not needed)
 // it splits K where the blocks do not fill the CUs evenly.
 bool skinny_fits(int64_t rows, int64_t columns, int64_t inner, int64_t lda, bool pair);
+// Whether the decode kernel comes first (where it fits).
+bool decode_before_skinny(int64_t rows, int64_t columns, int64_t inner, bool pair);
 size_t skinny_workspace_bytes(int64_t rows, int64_t columns, int64_t inner, int nw);
 hipError_t launch_q4_skinny(const splosh_q4_weight &w, const splosh_q4_weight *up, const uint16_t *a, int64_t lda,
                             void *out, int64_t ldc, int out_dtype, const void *residual, int64_t rows, void *workspace,

@@ -371,6 +371,15 @@ bool skinny_fits(int64_t rows, int64_t columns, int64_t inner, int64_t lda, bool
            (blocks <= cus && inner / kGroup < kSkinnyLong * 8);
 }
 
+// The calls of up to four rows that stay on the decode kernel where it takes them: one and two rows, and one
+// weight of at most half a block a CU with K1280 or K1536 (us, decode / here: three rows of K1536 -> N2048 4.0 /
+// 4.4, N512 3.8 / 3.9; but K1024 -> N2048 4.0 / 3.45, K1792 5.0 / 4.4, and K1536 -> N4608 5.1 / 4.55; the pair of
+// K1536 -> 2 x N2048 is level).
+bool decode_before_skinny(int64_t rows, int64_t columns, int64_t inner, bool pair) {
+    const int64_t groups = inner / kGroup;
+    return rows <= 2 || (rows <= 4 && !pair && 2 * (columns / kSkinnyCols) <= device_cus() && groups > 16 && groups <= 24);
+}
+
 static size_t skinny_need(const SkinnyPlan &p, int64_t rows, int nw) {
     if (p.split.slices < 2) return 0;
     const int rm = skinny_rows(rows), e = rm / 2;
