@@ -107,6 +107,8 @@ bool mma_fits(int64_t rows, int64_t columns, int64_t inner, int64_t stride_words
 // `unit_elems`: K elements of one unit (64 for q4 groups, 256 for Q5_K blocks).
 MmaPlan plan_mma(int64_t rows, int64_t columns, int64_t groups, bool mlp, size_t workspace_bytes,
                  int64_t unit_elems = 64);
+// Whether its workgroups take whole bands (no split over K) of the shape, given scratch.
+bool mma_whole_bands(int64_t rows, int64_t columns, int64_t groups, int64_t unit_elems);
 size_t mma_workspace_bytes(int64_t rows, int64_t columns, int64_t groups, bool mlp);
 hipError_t launch_q4_mma_group(const MmaPlan &plan, const splosh_q4_weight *w, int count, void *const *outs,
                                const int64_t *ldcs, const uint16_t *a, int64_t lda, int out_dtype, int64_t rows,

@@ -1293,6 +1293,10 @@ MmaPlan plan_mma(int64_t rows, int64_t columns, int64_t groups, bool mlp, size_t
     return p;
 }
 
+bool mma_whole_bands(int64_t rows, int64_t columns, int64_t groups, int64_t unit_elems) {
+    return plan_mma(rows, columns, groups, false, (size_t)-1, unit_elems).sk_units == 0;
+}
+
 size_t mma_workspace_bytes(int64_t rows, int64_t columns, int64_t groups, bool mlp) {
     const MmaPlan p = plan_mma(rows, columns, groups, mlp, (size_t)-1);
     return p.sk_units > 0 ? sk_bytes(p.grid, rows, p.bands, mlp) : 0;

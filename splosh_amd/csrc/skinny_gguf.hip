@@ -211,9 +211,25 @@ static bool sg_shape(int64_t rows, int64_t columns, int64_t inner, int64_t lda) 
 // the line, on mma.hip 11.0 and 11.9) and four of IQ4_NL, from 2048 blocks x units; 17 to 32 rows, where
 // the activations' traffic grows, of the types whose loads weigh most in mma.hip (32 rows: Q6_K 39.2 /
 // 43.2, Q3_K 31.8 / 46.3, IQ3_S 35.4 / 42.8, IQ4_XS in the file's order 32.3 / 34.1; not Q8_0 41.0 / 38.6).
+// Not between one and two blocks a CU, where a last round of workgroups leaves CUs idle, of the types that cost
+// mma.hip the least, from the rows at which it is the faster: where its bands come out whole (us, here / there: Q5_K 16
+// rows of K4096 -> N14336 15.4 / 14.7, of K1536 -> N12288 8.9 / 7.8 and at 7 rows 8.0 / 7.7; Q8_0 in the ROWS32 order 9 rows
+// of K4096 -> N12288 16.3 / 15.0, in the file's 19.3 / 21.6 but of K1536 10.5 / 9.1; IQ4_XS in the file's order 24 rows of
+// K1536 10.4 / 9.1), and at long K (K8192 -> N9216, 16 rows: Q5_K 25.2 / 22.2, Q8_0 43 / 34).
+static bool sg_uneven(int type, bool rows32, int64_t rows, int64_t columns, int64_t inner) {
+    const int64_t cus = device_cus(), blocks = (columns + kSgCols - 1) / kSgCols, units = inner / 256;
+    if (blocks <= cus || blocks >= 2 * cus) return false;
+    const bool shortk = units < 8, longk = units >= kSgLong;
+    int64_t from = 33;
+    if (type == 12 || type == 13) from = shortk ? 1 : longk ? 9 : 13;
+    else if (type == 8) from = shortk || longk ? 1 : rows32 ? 9 : 33;
+    else if ((type == 20 || type == 23) && shortk) from = type == 23 && !rows32 ? 17 : 9;
+    return rows >= from && (longk || mma_whole_bands(rows, columns, units, 256));
+}
 bool gguf_skinny_fits(int type, int64_t rows, int64_t columns, int64_t inner, int64_t lda, int64_t weight_bytes) {
     if (!sg_shape(rows, columns, inner, lda) || weight_bytes >= (int64_t)kSgOut - 65536) return false;
     const bool rows32 = gguf_layout(type);
+    if (sg_uneven(type, rows32, rows, columns, inner)) return false;
     if (rows <= 4) return rows > 1 && (columns + kSgCols - 1) / kSgCols * (inner / 256) >= 2048;
     return rows <= 16 || type == 14 || type == 11 || type == 21 || (type == 23 && !rows32);
 }

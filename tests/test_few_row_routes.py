@@ -13,10 +13,17 @@ LIB = wc.ROOT / "splosh_amd" / "libsplosh_q4.so"
 DECODE = [(f"decode_before_skinny({rows}, {n}, {k}, {pair})", want) for rows, n, k, pair, want in [
     (2, 17408, 5120, 0, 1), (2, 512, 1536, 1, 1), (3, 4096, 1536, 0, 1), (4, 128, 1280, 0, 1), (5, 512, 1536, 0, 0),
     (3, 4096, 1024, 0, 0), (3, 4096, 1792, 0, 0), (3, 4224, 1536, 0, 0), (4, 2048, 1536, 1, 0)]]
+# (type, rows, columns, inner): does the barrier-free GGUF kernel take it? (planes: 13 Q5_K, 12 Q4_K)
+GGUF = [(f"gguf_skinny_fits({kind}, {rows}, {n}, {k}, {k}, 1 << 20)", want) for kind, rows, n, k, want in [
+    (13, 16, 12288, 4096, 0), (12, 12, 14336, 2048, 1), (12, 13, 14336, 2048, 0), (13, 8, 12288, 1536, 0),
+    (13, 16, 8192, 1536, 1), (13, 16, 17408, 1536, 1), (13, 16, 9216, 4096, 1), (8, 7, 9216, 8192, 0),
+    (13, 8, 9216, 8192, 1), (13, 16, 9216, 8192, 0), (8, 16, 11008, 1536, 0), (8, 16, 12288, 4096, 1),
+    (8 | 0x100, 16, 12288, 4096, 0), (23, 16, 12288, 1536, 1), (23, 17, 12288, 1536, 0), (23, 17, 12288, 4096, 1),
+    (20, 8, 9216, 1536, 1), (20, 9, 9216, 1536, 0), (14, 16, 12288, 1536, 1), (11, 32, 12288, 4096, 1)]]
 
 
 @pytest.mark.skipif(not Path(wc.HIPCC).exists() or not LIB.exists(), reason="needs hipcc and the built library")
-@pytest.mark.parametrize("checks", [DECODE], ids=["decode"])
+@pytest.mark.parametrize("checks", [DECODE, GGUF], ids=["decode", "gguf"])
 def test_routes(tmp_path, checks):
     source, program = tmp_path / "routes.cpp", tmp_path / "routes"
     lines = "\n".join(f'    printf("%d\\n", (int)({e}));' for e, _ in checks)
