@@ -66,8 +66,9 @@ typedef enum splosh_dtype { SPLOSH_F32 = 0, SPLOSH_BF16 = 1 } splosh_dtype;
 typedef enum splosh_kernel {
     SPLOSH_KERNEL_AUTO = 0,     /* by layout, rows and size.
                                    TILED128: 1-2 rows STREAM (their staged activations fit 80 KB, K
-                                   up to about 18700); 3-16 rows, and 17-32 where it is the faster,
-                                   the raw-code MFMA kernel (skinny.hip); else up to 64 DEQUANT (a
+                                   up to about 18700), as a few shapes of 3-4; 3-16 rows, and 17-32
+                                   where it is the faster, the raw-code MFMA kernel (skinny.hip);
+                                   else up to 64 DEQUANT (a
                                    wide single weight as the pair of its column halves); 65-128 two
                                    calls of those, or PREFILL from 80 rows of a weight of 80 Mi
                                    elements given its scratch, or with the emit TILE or PREFILL;
@@ -255,8 +256,8 @@ int splosh_untile128(const void *src, void *dst, int64_t rows, int64_t groups, i
 
 /* Engine.gemm on a GGUF weight (Runtime/Engine.swift:1671-1697, kernels
  * Shaders/engine_gguf.metal:82-221 instantiated _q5k at :332-349). AUTO: one row takes the
- * every-CU decode kernel; 5..16 rows (2..4 of the larger weights) the barrier-free MFMA kernel of
- * skinny_gguf.hip, else up to 64 rows the stream-K one (DEQUANT), both on weights dequantized to bf16
+ * every-CU decode kernel; 5..16 rows (2..4 of the larger weights) mostly the barrier-free MFMA kernel
+ * of skinny_gguf.hip, else up to 64 rows the stream-K one (DEQUANT), both on weights dequantized to bf16
  * (lda % 8 == 0 and 16-byte aligned activations); 65..128 rows two calls of at most 64; more rows the
  * prefill kernel (PREFILL; also ldc % 4 == 0 and 16-byte aligned outputs), else the LDS-tiled kernel
  * (TILE), else the streaming kernel (STREAM). The MFMA kernels use a workspace of
